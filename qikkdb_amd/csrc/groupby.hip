@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "groupby.hpp"
+#include "ldstable.hpp"
 #include "lookback.hpp"
 #include "twophase.hpp"
 
@@ -32,152 +33,88 @@ namespace {
 
 constexpr int kSteps = 4;        // rows per thread per tile
 constexpr uint64_t kMaxLogical = (uint64_t)1 << 30;  // GB_BUFFER_SIZE_MAX (IGroupBy.h:6)
-constexpr int kLdsProbes = 8;    // LDS probe limit before a row goes to the global table
 constexpr int kEmitBlock = 256;
 constexpr int kEmitSteps = 16;
 constexpr int kEmitTile = kEmitBlock * kEmitSteps;
 
-// ---- LDS table of the one-pass kernel ----------------------------------------------------
-// Arrays of H hashed slots + 2 side slots (NULL key, key == kEmpty).
-struct Lds {
-    uint64_t* key;
-    uint64_t* sum;
-    uint64_t* mn;
-    uint64_t* mx;
-    uint32_t* cnt;
-    uint32_t* cntall;
-    int32_t H;
-};
-
-__host__ __device__ __forceinline__ int lds_slot_bytes(uint32_t fields) {
-    return 8 + 4 + ((fields & F_CNTALL) ? 4 : 0) + ((fields & F_SUM) ? 8 : 0) +
-           ((fields & F_MIN) ? 8 : 0) + ((fields & F_MAX) ? 8 : 0);
-}
-
-__device__ __forceinline__ Lds lds_carve(void* base, int32_t H, uint32_t fields) {
-    Lds t;
-    const int T = H + 2;
-    char* p = (char*)base;
-    t.key = (uint64_t*)p; p += (size_t)T * 8;
-    t.sum = (fields & F_SUM) ? (uint64_t*)p : nullptr; p += (fields & F_SUM) ? (size_t)T * 8 : 0;
-    t.mn = (fields & F_MIN) ? (uint64_t*)p : nullptr; p += (fields & F_MIN) ? (size_t)T * 8 : 0;
-    t.mx = (fields & F_MAX) ? (uint64_t*)p : nullptr; p += (fields & F_MAX) ? (size_t)T * 8 : 0;
-    t.cnt = (uint32_t*)p; p += (size_t)T * 4;
-    t.cntall = (fields & F_CNTALL) ? (uint32_t*)p : nullptr;
-    t.H = H;
-    return t;
-}
-
-__device__ __forceinline__ int lds_find(const Lds& t, uint64_t key, bool knull, uint64_t h) {
-    if (knull) {
-        if (t.key[t.H] == 0ull) t.key[t.H] = 1ull;
-        return t.H;
-    }
-    if (key == kEmpty) {
-        if (t.key[t.H + 1] == 0ull) t.key[t.H + 1] = 1ull;
-        return t.H + 1;
-    }
-    uint32_t s = (uint32_t)(((h >> 32) * (uint64_t)(uint32_t)t.H) >> 32);
-#pragma unroll 1
-    for (int p = 0; p < kLdsProbes; p++) {
-        uint64_t cur = __hip_atomic_load(&t.key[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (cur == key) return (int)s;
-        if (cur == kEmpty) {
-            unsigned long long old = atomicCAS((unsigned long long*)&t.key[s], (unsigned long long)kEmpty,
-                                               (unsigned long long)key);
-            if (old == kEmpty || old == key) return (int)s;
-        }
-        s = (s + 1 == (uint32_t)t.H) ? 0u : s + 1;
-    }
-    return -1;
-}
-
-template <bool REAL>
-__device__ __forceinline__ void lds_accum(const Lds& t, int s, const Part& p, uint32_t fields) {
-    if (p.cnt) atomicAdd(&t.cnt[s], (uint32_t)p.cnt);
-    if (fields & F_CNTALL) atomicAdd(&t.cntall[s], (uint32_t)p.cntall);
-    if (p.cnt) {
-        if (fields & F_SUM) {
-            if (REAL)
-                atomicAdd((double*)&t.sum[s], __longlong_as_double((long long)p.sum));
-            else
-                atomicAdd((unsigned long long*)&t.sum[s], (unsigned long long)p.sum);
-        }
-        if (fields & F_MIN) atomicMin((unsigned long long*)&t.mn[s], (unsigned long long)p.mn);
-        if (fields & F_MAX) atomicMax((unsigned long long*)&t.mx[s], (unsigned long long)p.mx);
-    }
-}
-
 // ---- the one-pass row kernel --------------------------------------------------------------
-// MODE 0: every row; 1: rows whose int8 mask is non-zero; 2: rows passing the predicates.
+// MODE 0: every row; 1: rows whose int8 mask is non-zero; 2: rows passing the predicates; 3 and 4:
+// a folded interval on the value column or on another column.
 // Row r of tile T is T*(kSteps*blockDim) + k*blockDim + threadIdx.x, so each step's loads
 // are coalesced spans.  Workgroups are persistent (grid-stride over tiles) so that the LDS
-// table sees many rows before it is merged.
+// table sees many rows before it is merged: into the global table with atomics, or, where every key
+// fits the LDS table, through `out` and k_gb_fold.
 template <int KW, typename VT, int MODE>
 __global__ void __launch_bounds__(1024) k_gb_rows(GView g, KeySpec ks, KeyCols kc,
                                                   const VT* __restrict__ vals,
                                                   const uint64_t* __restrict__ vnull,
                                                   const int8_t* __restrict__ mask, PredSet preds,
                                                   uint32_t vpred, int64_t n, uint32_t fields,
-                                                  int32_t H) {
+                                                  int32_t H, int32_t rbits, Partials out) {
     extern __shared__ uint64_t lds_raw[];
     __shared__ unsigned int s_new;
     constexpr bool HAS_V = VTraits<VT>::has;
     constexpr bool REAL = VTraits<VT>::real;
-    const bool use_lds = (KW == 1) && H > 0;
+    const bool use_lds = H > 0;
+    const int copy = threadIdx.x & ((1 << rbits) - 1);
     Lds t{};
     if (threadIdx.x == 0) s_new = 0;
     if (use_lds) {
-        t = lds_carve(lds_raw, H, fields);
-        for (int s = threadIdx.x; s < H + 2; s += blockDim.x) {
-            t.key[s] = s < H ? kEmpty : 0ull;
-            t.cnt[s] = 0;
-            if (t.cntall) t.cntall[s] = 0;
-            if (t.sum) t.sum[s] = 0;
-            if (t.mn) t.mn[s] = ~0ull;
-            if (t.mx) t.mx[s] = 0ull;
-        }
+        t = lds_carve(lds_raw, H, rbits, fields);
+        lds_clear(t);
     }
     __syncthreads();
 
     const int64_t bd = blockDim.x;
     const int64_t tile_rows = bd * kSteps;
     const int64_t ntiles = (n + tile_rows - 1) / tile_rows;
-    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    struct Tile {
         uint64_t key[kSteps][KW];
-        bool kn[kSteps], act[kSteps], vn[kSteps];
+        bool kn[kSteps], vn[kSteps], keep[kSteps], cn[kSteps];
+        int64_t cv[kSteps];
         typename std::conditional<HAS_V, VT, int>::type val[kSteps];
+    };
+    // rows past the end read the last row and are dropped: the loads are unconditional, so those of a
+    // tile are all in flight together
+    auto row_of = [&](int64_t tile, int k) { return tile * tile_rows + k * bd + threadIdx.x; };
+    auto load = [&](int64_t tile, Tile& T) {
+        int64_t r[kSteps];
+#pragma unroll
+        for (int k = 0; k < kSteps; k++) r[k] = min(row_of(tile, k), n - 1);
+        load_keys<KW, kSteps>(ks, kc, r, T.key, T.kn);
 #pragma unroll
         for (int k = 0; k < kSteps; k++) {
-            const int64_t r = tile * tile_rows + k * bd + threadIdx.x;
-            act[k] = r < n;
-            vn[k] = false;
-            kn[k] = false;
-            val[k] = {};
-            if (act[k]) {
-                load_key<KW>(ks, kc, r, key[k], kn[k]);
-                if constexpr (HAS_V) val[k] = vals[r];
-                vn[k] = vnull && null_bit(vnull, r);
-                if (MODE == 1) act[k] = mask[r] != 0;
-                if (MODE == 4)
-                    act[k] = !(preds.rnull && null_bit(preds.rnull, r)) && col_in_range(preds, range_col(preds, r));
+            T.val[k] = {};
+            if constexpr (HAS_V) T.val[k] = vals[r[k]];
+        }
+#pragma unroll
+        for (int k = 0; k < kSteps; k++) T.vn[k] = vnull && null_bit(vnull, r[k]);
+#pragma unroll
+        for (int k = 0; k < kSteps; k++) {
+            T.keep[k] = MODE == 1 ? mask[r[k]] != 0 : true;
+            T.cv[k] = 0;
+            T.cn[k] = false;
+            if (MODE == 4) {
+                T.cv[k] = range_col(preds, r[k]);
+                T.cn[k] = preds.rnull && null_bit(preds.rnull, r[k]);
             }
         }
-        if constexpr (MODE == 3 && HAS_V) {
+    };
+    auto process = [&](int64_t tile, const Tile& T) {
+        bool act[kSteps];
 #pragma unroll
-            for (int k = 0; k < kSteps; k++) act[k] = act[k] && !vn[k] && in_range<VT>(preds.vr, val[k]);
-        }
-        if (MODE == 2) {
-#pragma unroll
-            for (int k = 0; k < kSteps; k++) {
-                if (!act[k]) continue;
-                const int64_t r = tile * tile_rows + k * bd + threadIdx.x;
+        for (int k = 0; k < kSteps; k++) {
+            const int64_t r = row_of(tile, k);
+            act[k] = (r < n) & T.keep[k];
+            if (MODE == 4) act[k] = act[k] & !T.cn[k] & col_in_range(preds, T.cv[k]);
+            if constexpr (MODE == 3 && HAS_V) act[k] = act[k] & !T.vn[k] & in_range<VT>(preds.vr, T.val[k]);
+            if (MODE == 2 && act[k]) {
                 bool pass = true;
                 for (int p = 0; p < preds.n && pass; p++) {
                     const qk_predicate& q = preds.p[p];
                     if constexpr (HAS_V) {
                         if ((vpred >> p) & 1u) {
-                            pass = !vn[k] && pred_on_value(q, val[k], r);
+                            pass = !T.vn[k] && pred_on_value(q, T.val[k], r);
                             continue;
                         }
                     }
@@ -186,52 +123,70 @@ __global__ void __launch_bounds__(1024) k_gb_rows(GView g, KeySpec ks, KeyCols k
                 act[k] = pass;
             }
         }
+        // a multi-word key's slot: every row's home is read before any is compared
+        u64x2 tail[kSteps];
+        uint64_t home[kSteps];
+        if constexpr (KW > 1) {
+#pragma unroll
+            for (int k = 0; k < kSteps; k++) {
+                home[k] = home_of(g, key_hash<KW>(T.key[k]));
+                tail[k] = g_key_tail<KW>(g, home[k]);
+            }
+        }
 #pragma unroll
         for (int k = 0; k < kSteps; k++) {
             if (!act[k]) continue;
             Part p;
-            if constexpr (HAS_V) p = row_part<VT>(val[k], vn[k]); else p = row_part<NoValue>(NoValue{}, vn[k]);
-            const uint64_t h = key_hash<KW>(key[k]);
+            if constexpr (HAS_V) p = row_part<VT>(T.val[k], T.vn[k]); else p = row_part<NoValue>(NoValue{}, T.vn[k]);
             bool is_new = false;
             if constexpr (KW == 1) {
-                int ls = use_lds ? lds_find(t, key[k][0], kn[k], h) : -1;
+                const uint64_t h = hash64(T.key[k][0]);
+                int ls = use_lds ? lds_find(t, T.key[k][0], T.kn[k], h) : -1;
                 if (ls >= 0) {
-                    lds_accum<REAL>(t, ls, p, fields);
+                    lds_accum<REAL>(t, (ls << rbits) | copy, p, fields);
                 } else {
-                    const int64_t gs = g_slot1(g, key[k][0], kn[k], h, &is_new);
+                    const int64_t gs = g_slot1(g, T.key[k][0], T.kn[k], h, &is_new);
                     if (gs >= 0) g_accum_atomic(g, gs, p, fields); else g_set_lost(g);
                 }
             } else {
-                const int64_t gs = g_slotN<KW>(g, key[k], h, &is_new);
-                if (gs >= 0) g_accum_atomic(g, gs, p, fields); else g_set_lost(g);
+                int64_t gs = g_find_cached<KW>(g, T.key[k], home[k], tail[k]);
+                if (gs < 0) gs = g_slotN<KW>(g, T.key[k], key_hash<KW>(T.key[k]), &is_new);
+                if (gs < 0) {
+                    g_set_lost(g);
+                } else {
+                    const int ls = use_lds ? lds_find(t, (uint64_t)gs, false, hash64((uint64_t)gs)) : -1;
+                    if (ls >= 0) lds_accum<REAL>(t, (ls << rbits) | copy, p, fields);
+                    else g_accum_atomic(g, gs, p, fields);
+                }
             }
             if (is_new) atomicAdd(&s_new, 1u);
+        }
+    };
+    int64_t tile = blockIdx.x;
+    if constexpr (KW == 1 && MODE != 2) {
+        // the next tile's loads are issued before this tile is aggregated (two register sets)
+        Tile A, B;
+        if (tile < ntiles) load(tile, A);
+        while (tile < ntiles) {
+            load(tile + gridDim.x, B);
+            process(tile, A);
+            tile += gridDim.x;
+            if (tile >= ntiles) break;
+            load(tile + gridDim.x, A);
+            process(tile, B);
+            tile += gridDim.x;
+        }
+    } else {
+        for (; tile < ntiles; tile += gridDim.x) {
+            Tile A;
+            load(tile, A);
+            process(tile, A);
         }
     }
 
     if (use_lds) {
         __syncthreads();
-        for (int s = threadIdx.x; s < H + 2; s += blockDim.x) {
-            const uint64_t k = t.key[s];
-            if (s < H ? (k == kEmpty) : (k == 0ull)) continue;
-            Part p;
-            p.cnt = t.cnt[s];
-            p.cntall = t.cntall ? t.cntall[s] : 0;
-            p.sum = t.sum ? t.sum[s] : 0;
-            p.mn = t.mn ? t.mn[s] : ~0ull;
-            p.mx = t.mx ? t.mx[s] : 0ull;
-            bool is_new = false;
-            int64_t gs;
-            if (s == H) {
-                gs = g_slot1(g, 0ull, true, 0, &is_new);
-            } else if (s == H + 1) {
-                gs = g_slot1(g, kEmpty, false, 0, &is_new);
-            } else {
-                gs = g_slot1(g, k, false, hash64(k), &is_new);
-            }
-            if (is_new) atomicAdd(&s_new, 1u);
-            if (gs >= 0) g_accum_atomic(g, gs, p, fields); else g_set_lost(g);
-        }
+        lds_flush<KW, REAL>(t, g, out, fields, &s_new);
     }
     __syncthreads();
     if (threadIdx.x == 0) g_count_new(g, s_new);
@@ -573,11 +528,11 @@ __global__ void __launch_bounds__(256) k_gb_absent(GView g, KeySpec ks, KeyCols 
 template <int KW, typename VT, int MODE>
 int launch_rows_t(const GView& g, const KeySpec& ks, const KeyCols& kc, const void* vals,
                   const uint64_t* vnull, const int8_t* mask, const PredSet& ps, uint32_t vpred,
-                  int64_t n, uint32_t fields, int32_t H, int block, int wgs_per_cu,
+                  int64_t n, uint32_t fields, const LdsShape& L, int block, int wgs_per_cu,
                   hipStream_t s) {
     auto kern = k_gb_rows<KW, VT, MODE>;
     // gfx950 launches up to 160 KB of LDS per workgroup without a function attribute
-    const size_t lds = (KW == 1 && H > 0) ? (size_t)(H + 2) * lds_slot_bytes(fields) : 0;
+    const size_t lds = L.H > 0 ? lds_table_bytes(L.H, L.rbits, fields) : 0;
     int occ = 0;
     QK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, block, lds));
     if (occ < 1) return fail(QK_ERROR, "group by: launch shape (block %d, LDS %zu B) does not fit", block, lds);
@@ -585,26 +540,29 @@ int launch_rows_t(const GView& g, const KeySpec& ks, const KeyCols& kc, const vo
     const int64_t tile_rows = (int64_t)block * kSteps;
     const int64_t ntiles = (n + tile_rows - 1) / tile_rows;
     int64_t grid = (int64_t)device_info().cus * occ;
+    if (L.all) grid = std::min<int64_t>({grid, kMaxPartials, (n + L.min_rows - 1) / L.min_rows});
     if (grid > ntiles) grid = ntiles;
     if (grid < 1) grid = 1;
+    const Partials part = L.for_wgs(grid);
     kern<<<(unsigned)grid, block, lds, s>>>(g, ks, kc, (const VT*)vals, vnull, mask, ps, vpred, n,
-                                            fields, (KW == 1) ? H : 0);
+                                            fields, L.H, L.rbits, part);
     QK_HIP(hipGetLastError());
+    if (part.key) return fold_partials(g, L, (int32_t)grid, VTraits<VT>::real, fields, s);
     return QK_SUCCESS;
 }
 
 template <int KW, typename VT>
 int launch_rows_m(int mode, const GView& g, const KeySpec& ks, const KeyCols& kc, const void* vals,
                   const uint64_t* vnull, const int8_t* mask, const PredSet& ps, uint32_t vpred,
-                  int64_t n, uint32_t fields, int32_t H, int block, int wpc, hipStream_t s) {
+                  int64_t n, uint32_t fields, const LdsShape& L, int block, int wpc, hipStream_t s) {
     switch (mode) {
-    case 0: return launch_rows_t<KW, VT, 0>(g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, H, block, wpc, s);
-    case 1: return launch_rows_t<KW, VT, 1>(g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, H, block, wpc, s);
-    case 2: return launch_rows_t<KW, VT, 2>(g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, H, block, wpc, s);
-    case 4: return launch_rows_t<KW, VT, 4>(g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, H, block, wpc, s);
+    case 0: return launch_rows_t<KW, VT, 0>(g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, L, block, wpc, s);
+    case 1: return launch_rows_t<KW, VT, 1>(g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, L, block, wpc, s);
+    case 2: return launch_rows_t<KW, VT, 2>(g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, L, block, wpc, s);
+    case 4: return launch_rows_t<KW, VT, 4>(g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, L, block, wpc, s);
     default:
         if constexpr (VTraits<VT>::has)
-            return launch_rows_t<KW, VT, 3>(g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, H, block, wpc, s);
+            return launch_rows_t<KW, VT, 3>(g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, L, block, wpc, s);
         return fail(QK_ERROR, "value range filter without a value column");
     }
 }
@@ -612,14 +570,14 @@ int launch_rows_m(int mode, const GView& g, const KeySpec& ks, const KeyCols& kc
 template <int KW>
 int launch_rows_v(int vtype, int mode, const GView& g, const KeySpec& ks, const KeyCols& kc,
                   const void* vals, const uint64_t* vnull, const int8_t* mask, const PredSet& ps,
-                  uint32_t vpred, int64_t n, uint32_t fields, int32_t H, int block, int wpc,
+                  uint32_t vpred, int64_t n, uint32_t fields, const LdsShape& L, int block, int wpc,
                   hipStream_t s) {
-    if (!vals) return launch_rows_m<KW, NoValue>(mode, g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, H, block, wpc, s);
+    if (!vals) return launch_rows_m<KW, NoValue>(mode, g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, L, block, wpc, s);
     switch (vtype) {
-    case QK_INT: return launch_rows_m<KW, int32_t>(mode, g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, H, block, wpc, s);
-    case QK_LONG: return launch_rows_m<KW, int64_t>(mode, g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, H, block, wpc, s);
-    case QK_FLOAT: return launch_rows_m<KW, float>(mode, g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, H, block, wpc, s);
-    case QK_DOUBLE: return launch_rows_m<KW, double>(mode, g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, H, block, wpc, s);
+    case QK_INT: return launch_rows_m<KW, int32_t>(mode, g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, L, block, wpc, s);
+    case QK_LONG: return launch_rows_m<KW, int64_t>(mode, g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, L, block, wpc, s);
+    case QK_FLOAT: return launch_rows_m<KW, float>(mode, g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, L, block, wpc, s);
+    case QK_DOUBLE: return launch_rows_m<KW, double>(mode, g, ks, kc, vals, vnull, mask, ps, vpred, n, fields, L, block, wpc, s);
     default: return fail(QK_ERROR, "group by: unsupported value type %d", vtype);
     }
 }
@@ -657,6 +615,10 @@ struct qk_groupby_s {
     int32_t last_H = 0;
     int32_t last_path = 0;
     int64_t grows = 0;      // growths of a QK_GB_AUTO_GROW table
+    // the one-pass kernel's workgroup tables (partials_for): entries per array
+    uint64_t* part_buf = nullptr;
+    size_t part_words = 0;
+    hipStream_t part_stream = nullptr;  // that last used it
     // pre-seeded keys (GPUGroupBy(maxHashCount, keys, firstKeyIsNull)): their slots in seed
     // order and a bit per slot; GetResults emits them first, in that order
     int64_t* seed_slot = nullptr;
@@ -864,18 +826,70 @@ int grow_table(qk_groupby_s* h, uint64_t need, hipStream_t s) {
     return QK_SUCCESS;
 }
 
-int choose_lds_slots(const qk_groupby_s* h) {
-    if (h->ks.kw != 1 || h->lds_budget == 0) return 0;
+// The LDS table of the one-pass kernel: up to two slots per key the table may hold, within the
+// budget; states in as many copies (up to 32) as still fit beside that many slots.
+LdsShape choose_lds(const qk_groupby_s* h) {
+    LdsShape L;
+    if (h->lds_budget == 0) return L;
     const DeviceInfo& d = device_info();
     size_t budget = h->lds_budget > 0 ? (size_t)h->lds_budget : d.lds_per_cu / 2;
     if (budget > d.lds_per_block) budget = d.lds_per_block;
-    const int bps = lds_slot_bytes(h->fields);
-    int64_t slots = (int64_t)(budget / (size_t)bps) - 2;
-    // no point holding more LDS slots than twice the table's key capacity
-    const int64_t useful = (int64_t)std::min<uint64_t>(h->logical_cap * 2 + 64, (uint64_t)1 << 30);
-    if (slots > useful) slots = useful;
-    if (slots < 64) return 0;
-    return (int)slots;
+    const int64_t fits = (int64_t)(budget / lds_table_bytes(-1, 0, h->fields)) - 2;
+    // no point holding more LDS slots than two per key of the table's capacity (a power of two, whose
+    // home slots the small-table kernel takes by a shift)
+    int64_t useful = 64;
+    while (useful < 2 * (int64_t)h->logical_cap) useful <<= 1;
+    const int64_t slots = std::min(fits, useful);
+    if (slots < 64) return L;
+    L.H = (int32_t)slots;
+    if (fits >= useful) {
+        while (L.rbits < kMaxCopyBits && lds_table_bytes(L.H, L.rbits + 1, h->fields) <= budget) L.rbits++;
+        L.all = true;
+        L.keys = (int64_t)h->logical_cap;
+        // two rows per entry: a workgroup's table then costs no more traffic than its rows
+        L.min_rows = 2 * (int64_t)L.H;
+    }
+    return L;
+}
+
+// Memory for the workgroups' tables, kept with the table.  Without it (no memory left, or a first
+// block under graph capture, where nothing can be allocated) they go straight to the global table;
+// so do those of an asynchronous table's blocks on another stream than the first, which may run
+// while that one's use it.
+void partials_for(qk_groupby_s* h, LdsShape* L, hipStream_t s) {
+    if ((h->flags & QK_GB_ASYNC) && h->part_buf && h->part_stream != s) return;
+    const size_t words = (size_t)kMaxPartials * (size_t)(L->H + 2);
+    int arrays = 2;
+    for (uint32_t f : {F_CNTALL, F_SUM, F_MIN, F_MAX}) arrays += (h->fields & f) ? 1 : 0;
+    if (h->part_words < words) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return;
+        }
+        if (h->part_buf) {
+            // another stream's last block may still use the smaller one
+            if (hipDeviceSynchronize() != hipSuccess) return;
+            pool_free(h->part_buf);
+            h->part_buf = nullptr;
+            h->part_words = 0;
+        }
+        if (pool_alloc((void**)&h->part_buf, words * 8 * (size_t)arrays) != QK_SUCCESS) return;
+        h->part_words = words;
+    }
+    h->part_stream = s;
+    uint64_t* p = h->part_buf;
+    auto next = [&](bool on) {
+        uint64_t* at = on ? p : nullptr;
+        if (on) p += h->part_words;
+        return at;
+    };
+    L->part.key = next(true);
+    L->part.cnt = next(true);
+    L->part.cntall = next(h->fields & F_CNTALL);
+    L->part.sum = next(h->fields & F_SUM);
+    L->part.mn = next(h->fields & F_MIN);
+    L->part.mx = next(h->fields & F_MAX);
 }
 
 std::pair<hipEvent_t, hipEvent_t>* next_events(qk_groupby h) {
@@ -920,8 +934,11 @@ int process_once(qk_groupby h, int mode, const void* const* keys, const uint64_t
     GView g = view_of(h);
     std::pair<hipEvent_t, hipEvent_t>* ev = h->profiling ? next_events(h) : nullptr;
     const int vtype = values ? h->value_type : 0;
+    // a table whose every key fits a workgroup's LDS takes the one-pass kernel at any size
+    LdsShape L = choose_lds(h);
     const bool two = twophase_supported(h->ks.kw, h->value_type) &&
-                     (h->twophase_mode == 1 || (h->twophase_mode < 0 && n >= h->twophase_min_rows));
+                     (h->twophase_mode == 1 ||
+                      (h->twophase_mode < 0 && n >= h->twophase_min_rows && !L.all));
     int st;
     if (two) {
         // Phase 2 is deferred across blocks only for asynchronous tables: a synchronous table
@@ -942,14 +959,15 @@ int process_once(qk_groupby h, int mode, const void* const* keys, const uint64_t
                              h->fields, mode, s, ev ? ev->first : nullptr, ev ? ev->second : nullptr);
         if (st == QK_SUCCESS && !defer) st = twophase_flush(tp, g, h->fields, s);
     } else {
-        const int32_t H = choose_lds_slots(h);
-        h->last_H = H;
+        if (L.all) partials_for(h, &L, s);
+        h->last_H = L.H;
         h->last_path = 0;
         if (ev) QK_HIP(hipEventRecord(ev->first, s));
-        switch (h->ks.kw) {
-        case 1: st = launch_rows_v<1>(vtype, mode, g, h->ks, kc, values, value_nulls, mask, ps, vpred, n, h->fields, H, h->block, h->wgs_per_cu, s); break;
-        case 2: st = launch_rows_v<2>(vtype, mode, g, h->ks, kc, values, value_nulls, mask, ps, vpred, n, h->fields, 0, h->block, h->wgs_per_cu, s); break;
-        default: st = launch_rows_v<4>(vtype, mode, g, h->ks, kc, values, value_nulls, mask, ps, vpred, n, h->fields, 0, h->block, h->wgs_per_cu, s); break;
+        switch (small_supported(h->ks, kc, mode, n, L) ? 0 : h->ks.kw) {
+        case 0: st = small_rows(g, h->ks, kc, vtype, values, value_nulls, ps, mode, n, h->fields, L, s); break;
+        case 1: st = launch_rows_v<1>(vtype, mode, g, h->ks, kc, values, value_nulls, mask, ps, vpred, n, h->fields, L, h->block, h->wgs_per_cu, s); break;
+        case 2: st = launch_rows_v<2>(vtype, mode, g, h->ks, kc, values, value_nulls, mask, ps, vpred, n, h->fields, L, h->block, h->wgs_per_cu, s); break;
+        default: st = launch_rows_v<4>(vtype, mode, g, h->ks, kc, values, value_nulls, mask, ps, vpred, n, h->fields, L, h->block, h->wgs_per_cu, s); break;
         }
         if (st == QK_SUCCESS && ev) QK_HIP(hipEventRecord(ev->second, s));
     }
@@ -1044,7 +1062,7 @@ int collect_profile(qk_groupby h) {
 }
 
 void free_table(qk_groupby_s* h) {
-    void* ptrs[] = {h->keys, h->cnt, h->cntall, h->sum, h->mn, h->mx, h->ctr, h->seed_slot, h->seed_bits};
+    void* ptrs[] = {h->keys, h->cnt, h->cntall, h->sum, h->mn, h->mx, h->ctr, h->seed_slot, h->seed_bits, h->part_buf};
     for (void* p : ptrs)
         if (p) pool_free(p);
     twophase_free(h->tp);

@@ -154,6 +154,71 @@ __device__ __forceinline__ void load_key(const KeySpec& ks, const KeyCols& kc, i
     if (KW > 1) k[KW - 1] |= kPresent;
 }
 
+// The key words of N rows, every row's load of a column issued before any is used (the type
+// switch is outside the row loop, so a wave waits once per column and not once per row).
+template <int KW, int N>
+__device__ __forceinline__ void load_keys(const KeySpec& ks, const KeyCols& kc, const int64_t (&r)[N],
+                                          uint64_t (&k)[N][KW], bool (&kn)[N]) {
+    const bool single = KW == 1 && ks.single;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        kn[i] = false;
+#pragma unroll
+        for (int w = 0; w < KW; w++) k[i][w] = 0;
+    }
+    for (int c = 0; c < (single ? 1 : ks.nkeys); c++) {
+        bool isnull[N];
+        if (kc.nm[c]) {
+#pragma unroll
+            for (int i = 0; i < N; i++) isnull[i] = null_bit(kc.nm[c], r[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < N; i++) isnull[i] = false;
+        }
+        uint64_t f[N];
+        const int type = ks.type[c];
+        if (type == QK_INT || type == QK_FLOAT) {
+            uint32_t x[N];
+#pragma unroll
+            for (int i = 0; i < N; i++) x[i] = to_g((const uint32_t*)kc.col[c])[r[i]];
+#pragma unroll
+            for (int i = 0; i < N; i++)
+                f[i] = type == QK_FLOAT ? fkey32(__uint_as_float(x[i]))
+                                        : (single ? (uint64_t)(int64_t)(int32_t)x[i] : (uint64_t)x[i]);
+        } else if (type == QK_LONG || type == QK_DOUBLE) {
+#pragma unroll
+            for (int i = 0; i < N; i++) f[i] = to_g((const uint64_t*)kc.col[c])[r[i]];
+            if (type == QK_DOUBLE) {
+#pragma unroll
+                for (int i = 0; i < N; i++) f[i] = fkey64(__longlong_as_double((long long)f[i]));
+            }
+        } else {
+            int8_t x[N];
+#pragma unroll
+            for (int i = 0; i < N; i++) x[i] = to_g((const int8_t*)kc.col[c])[r[i]];
+#pragma unroll
+            for (int i = 0; i < N; i++) f[i] = single ? (uint64_t)(int64_t)x[i] : (uint64_t)(uint32_t)(int32_t)x[i];
+        }
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            if (single) {
+                k[i][0] = isnull[i] ? 0ull : f[i];
+                kn[i] = isnull[i];
+                continue;
+            }
+            // a NULL column contributes its null flag (composite keys of one word carry none)
+            const uint64_t v = isnull[i] ? (KW > 1 ? 1ull << ks.nshift[c] : 0ull) : f[i] << ks.shift[c];
+            const int at = isnull[i] ? ks.nword[c] : ks.word[c];
+#pragma unroll
+            for (int w = 0; w < KW; w++) k[i][w] |= w == at ? v : 0ull;
+        }
+    }
+    if (KW > 1) {
+#pragma unroll
+        for (int i = 0; i < N; i++) k[i][KW - 1] |= kPresent;
+    }
+}
+
 template <int KW>
 __device__ __forceinline__ uint64_t key_hash(const uint64_t (&k)[KW]) {
     uint64_t h = hash64(k[0]);
@@ -272,6 +337,40 @@ __device__ __forceinline__ int64_t g_slot1_claim(const GView& g, uint64_t key, u
     return -1;
 }
 
+// Two key words read by one 16-byte load.
+typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+template <int KW>
+__device__ __forceinline__ u64x2 g_key_tail(const GView& g, uint64_t s) {
+    return ((gptr<const u64x2>)(g.keys + s * KW))[KW / 2 - 1];
+}
+
+// Slot of a multi-word key the table already holds, through the caches: `tail` is slot `s`'s last
+// two words (s the key's home).  -1 means "not seen here", and the caller asks g_slotN: an empty or
+// busy word may be a stale copy.  A match is never stale: a stored key does not change, and the 16
+// bytes come from one copy of one line, in which the last word (written last, with release order)
+// is not newer than the word beside it.  A four-word key's first half is read after its last half
+// has matched, so from the same copy of the line or a newer one.
+template <int KW>
+__device__ __forceinline__ int64_t g_find_cached(const GView& g, const uint64_t (&k)[KW], uint64_t s, u64x2 tail) {
+    constexpr int kProbes = 4;
+#pragma unroll 1
+    for (int p = 0;; p++) {
+        if (tail.y == 0ull || tail.y == kBusy) return -1;
+        bool eq = (tail.y == k[KW - 1]) & (tail.x == k[KW - 2]);
+        if constexpr (KW == 4) {
+            if (eq) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                const u64x2 head = ((gptr<const u64x2>)(g.keys + s * KW))[0];
+                eq = (head.x == k[0]) & (head.y == k[1]);
+            }
+        }
+        if (eq) return (int64_t)s;
+        if (p + 1 == kProbes) return -1;
+        s = next_in_sub(g, s);
+        tail = g_key_tail<KW>(g, s);
+    }
+}
+
 // Slot of a multi-word key: the last word is claimed (0 -> kBusy), the other words written,
 // then the last word published with release order; readers that see kBusy wait for it.
 template <int KW>
@@ -340,7 +439,10 @@ __device__ __forceinline__ bool g_hasN(const GView& g, const uint64_t (&k)[KW], 
     return false;
 }
 
-// Atomic merge of a partial into slot s (concurrent writers allowed).
+// Atomic merge of a partial into slot s (concurrent writers allowed).  READ: minima and maxima are
+// read first, which skips the atomics that cannot change the value (worth it per row; a merge of few
+// entries rather saves the round trip).
+template <bool READ = true>
 __device__ __forceinline__ void g_accum_atomic(const GView& g, int64_t s, const Part& p, uint32_t fields) {
     if (p.cnt) g_atomic_add((unsigned long long*)(g.cnt + s), (unsigned long long)p.cnt);
     if ((fields & F_CNTALL) && p.cntall) g_atomic_add((unsigned long long*)(g.cntall + s), (unsigned long long)p.cntall);
@@ -351,10 +453,9 @@ __device__ __forceinline__ void g_accum_atomic(const GView& g, int64_t s, const 
             else
                 g_atomic_add((unsigned long long*)(g.sum + s), (unsigned long long)p.sum);
         }
-        // the read first skips atomics that cannot change the value
-        if ((fields & F_MIN) && p.mn < g_load_volatile(g.mn + s))
+        if ((fields & F_MIN) && (!READ || p.mn < g_load_volatile(g.mn + s)))
             g_atomic_min((unsigned long long*)(g.mn + s), (unsigned long long)p.mn);
-        if ((fields & F_MAX) && p.mx > g_load_volatile(g.mx + s))
+        if ((fields & F_MAX) && (!READ || p.mx > g_load_volatile(g.mx + s)))
             g_atomic_max((unsigned long long*)(g.mx + s), (unsigned long long)p.mx);
     }
 }

@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "rowstream.hpp"
 #include "twophase.hpp"
 
 namespace qk {
@@ -47,35 +48,6 @@ __device__ __forceinline__ void get_rec(const uint32_t* base, int64_t at, uint64
     const typename R::Rec r = *reinterpret_cast<const typename R::Rec*>(base + at * R::words);
     key = (uint64_t)r.w[0] | ((uint64_t)r.w[1] << 32);
     if constexpr (VTraits<VT>::has) __builtin_memcpy(&v, &r.w[2], sizeof(VT)); else v = 0;
-}
-
-// VV is VT, or a placeholder type when the table reads no value column.  MODE: 0 no WHERE,
-// 1 row mask, 2 predicate list, 3 folded interval on the value column, 4 folded interval on
-// another integer column, whose value (cv) and NULL bit (cn) the caller loaded.
-template <typename VT, int MODE, typename VV>
-__device__ __forceinline__ bool row_passes(const PredSet& preds, uint32_t vpred, const int8_t* mask,
-                                           int64_t r, const VV& v, bool vn, int64_t cv = 0, bool cn = false) {
-    if (MODE == 1) return mask[r] != 0;
-    // & rather than &&: both sides are cheap and side-effect free, and a short circuit would
-    // become a divergent branch per row
-    if constexpr (MODE == 3 && VTraits<VT>::has) return !vn & in_range<VT>(preds.vr, v);
-    if (MODE == 4) return !cn & col_in_range(preds, cv);
-    if (MODE == 2) {
-        for (int p = 0; p < preds.n; p++) {
-            const qk_predicate& q = preds.p[p];
-            bool pass;
-            if constexpr (VTraits<VT>::has) {
-                if ((vpred >> p) & 1u)
-                    pass = !vn && pred_on_value(q, v, r);
-                else
-                    pass = eval_pred(q, r);
-            } else {
-                pass = eval_pred(q, r);
-            }
-            if (!pass) return false;
-        }
-    }
-    return true;
 }
 
 // Exclusive prefix sum over the threads of a workgroup (blockDim a multiple of 64, <= 1024);
@@ -457,23 +429,8 @@ __device__ __forceinline__ int heavy_find(const uint64_t* lkey, uint32_t nb, uin
     return s;
 }
 
-// KT is the element type of a single integer key column, KeyPairI32 for two non-NULL int32
-// key columns packed into one word (the first in the low half), or void for any key layout
-// (read through the key spec's runtime switch).  With a typed key, the loads of a whole tile
-// are issued before any of them is used.
-struct KeyPairI32 {};
-template <typename KT>
-constexpr bool kPairKey = std::is_same<KT, KeyPairI32>::value;
-template <typename KT>
-constexpr bool kTypedKey = !std::is_same<KT, void>::value && !kPairKey<KT>;
-
 // The global table is read through a pointer: only the rare atomic path needs it, and kernel
 // arguments kept in scalar registers for the whole loop would spill.
-//
-// FP selects the aggregate states the LDS table keeps: kFieldsSum fixes them at sum + count
-// (SUM, AVG, COUNT; no MIN/MAX) so that the loop carries no per-field tests; kFieldsAny reads
-// them from `fields`.
-constexpr int kFieldsAny = 0, kFieldsSum = 1;
 
 // The phase-1 LDS of one workgroup, carved as p1_lds_bytes lays it out.
 template <typename VV>
@@ -796,87 +753,8 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase1(const GView* gp, KeySpec k
 
 // ---- phase 1, streaming form ----------------------------------------------------------------
 //
-// The same work as k_tp_phase1 for one typed key column (int32 or int64, nullable) or two
-// non-NULL int32 key columns packed into one word, with no WHERE or a WHERE folded into an
-// interval (on the value column or on one other integer column).  A wavefront takes chunks of
-// kSChunk rows in parts of kSPart rows; lane l holds rows 2l and 2l+1 of every part, so every
-// load instruction reads one contiguous 512 B (4-byte column) or 1 KB (8-byte column) range
-// with 8- or 16-byte lanes, and a null bitmap costs one 32-bit load per part.  The loads are
-// buffer loads bounded by the resource's size: rows past the end read as zero and an absent
-// bitmap is a resource of size zero, so no load needs a bounds
-// test or a clamp, and the next chunk's loads are issued before the current chunk is
-// aggregated.  Offsets are 32-bit bytes: every column of the block stays below 2^31 bytes.
-
-constexpr int kSRows = 4;                 // rows per lane per chunk
-constexpr int kSParts = kSRows / 2;        // parts of a chunk: lane l holds rows 2l, 2l+1 of each
-constexpr int kSChunk = 64 * kSRows;      // rows per wavefront per chunk
-constexpr int kSPart = 128;               // rows per part
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, int64_t bytes) {
-    // word 3 = 0x00020000: the untyped 32-bit data format of raw buffer accesses on gfx9
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
-}
-
-// The 32-bit words of one lane's kSRows rows of a column of E-byte elements: row j of the lane
-// in w[j] (E = 4) or w[2j], w[2j+1] (E = 8).
-template <int E>
-struct LaneWords {
-    uint32_t w[E * kSRows / 4];
-};
-
-// Every part of a lane's rows, the first at byte offset off, the next kSPart * E bytes further
-// each (non-temporal: the columns are streamed once, and the lines of the cold regions being
-// filled should stay in the L2).
-__device__ __forceinline__ void ld_lane(__amdgpu_buffer_rsrc_t r, uint32_t off, LaneWords<4>& t) {
-#pragma unroll
-    for (int q = 0; q < kSParts; q++) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)(off + q * kSPart * 4), 0, 2);
-        t.w[2 * q] = v[0];
-        t.w[2 * q + 1] = v[1];
-    }
-}
-__device__ __forceinline__ void ld_lane(__amdgpu_buffer_rsrc_t r, uint32_t off, LaneWords<8>& t) {
-#pragma unroll
-    for (int q = 0; q < kSParts; q++) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off + q * kSPart * 8), 0, 2);
-        t.w[4 * q] = v[0];
-        t.w[4 * q + 1] = v[1];
-        t.w[4 * q + 2] = v[2];
-        t.w[4 * q + 3] = v[3];
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ T word_elem(const uint32_t* w, int j) {
-    if constexpr (sizeof(T) == 8) {
-        const uint64_t u = (uint64_t)w[2 * j] | ((uint64_t)w[2 * j + 1] << 32);
-        return __builtin_bit_cast(T, u);
-    } else {
-        return __builtin_bit_cast(T, w[j]);
-    }
-}
-
-// A null bitmap's words for every part of a lane's rows: the lane's two rows of a part lie in
-// one 32-bit word (2l is even), each part's word kSPart / 32 words after the previous one's.
-struct LaneBits {
-    uint32_t w[kSParts];
-    __device__ __forceinline__ bool bit(int j, uint32_t sh) const {
-        return (w[j >> 1] >> (sh + (uint32_t)(j & 1))) & 1u;
-    }
-};
-__device__ __forceinline__ LaneBits no_bits() {
-    LaneBits b;
-#pragma unroll
-    for (int q = 0; q < kSParts; q++) b.w[q] = 0u;
-    return b;
-}
-__device__ __forceinline__ LaneBits ld_bits(__amdgpu_buffer_rsrc_t r, uint32_t boff) {
-    LaneBits b;
-#pragma unroll
-    for (int q = 0; q < kSParts; q++)
-        b.w[q] = __builtin_amdgcn_raw_buffer_load_b32(r, (int)(boff + q * (kSPart / 8)), 0, 0);
-    return b;
-}
+// The same work as k_tp_phase1 over the rows of stream_rows (rowstream.hpp): one typed key column or
+// two packed int32 columns, under no WHERE or a folded one.
 
 template <typename VT, int MODE, typename KT, int FP>
 __global__ void __launch_bounds__(kBlock) k_tp_phase1s(const GView* gp, KeyCols kc, const VT* __restrict__ vals,
@@ -884,126 +762,38 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase1s(const GView* gp, KeyCols 
                                                        int32_t n, uint32_t fields, P1Args a) {
     extern __shared__ __align__(16) uint64_t lds[];
     constexpr bool HAS_V = VTraits<VT>::has;
-    constexpr bool PAIR = kPairKey<KT>;
     using VV = typename std::conditional<HAS_V, VT, int>::type;
-    constexpr int KE = PAIR ? 4 : (int)sizeof(KT);          // bytes per row of a key column
-    constexpr int VE = HAS_V ? (int)sizeof(VV) : 4;         // bytes per row of the value column
     const bool f_sum = FP == kFieldsSum ? true : (fields & F_SUM) != 0;
     const bool f_min = FP == kFieldsSum ? false : (fields & F_MIN) != 0;
     const bool f_max = FP == kFieldsSum ? false : (fields & F_MAX) != 0;
-    const int H = a.H, tid = threadIdx.x;
-    const int lane = tid & 63;
+    const int H = a.H;
     const uint32_t nb = (uint32_t)(H / kBucket);
     const P1Lds<VV> L = p1_begin<VT, VV>(lds, a, f_sum, f_min, f_max);
     const int32_t K = __builtin_amdgcn_readfirstlane(min(a.meta[0], a.kmax));
-
-    const int64_t bitmap_bytes = ((int64_t)n + 63) / 64 * 8;
-    const __amdgpu_buffer_rsrc_t rk0 = make_rsrc(kc.col[0], (int64_t)n * KE);
-    const __amdgpu_buffer_rsrc_t rk1 = make_rsrc(PAIR ? kc.col[1] : kc.col[0], PAIR ? (int64_t)n * KE : 0);
-    const __amdgpu_buffer_rsrc_t rkn = make_rsrc(kc.nm[0], (!PAIR && kc.nm[0]) ? bitmap_bytes : 0);
-    const __amdgpu_buffer_rsrc_t rv = make_rsrc(vals, HAS_V ? (int64_t)n * VE : 0);
-    const __amdgpu_buffer_rsrc_t rvn = make_rsrc(vnull, vnull ? bitmap_bytes : 0);
-    const int CE = preds.rwide ? 8 : 4;
-    const __amdgpu_buffer_rsrc_t rc = make_rsrc(preds.rcol, MODE == 4 ? (int64_t)n * CE : 0);
-    const __amdgpu_buffer_rsrc_t rcn = make_rsrc(preds.rnull, (MODE == 4 && preds.rnull) ? bitmap_bytes : 0);
-
-    struct Chunk {
-        LaneWords<KE> k0, k1;
-        LaneWords<VE> v;
-        LaneWords<8> c;
-        LaneBits vb, kb, cb;
-    };
-    // the chunk's loads; a chunk past the end reads zeros
-    auto load = [&](uint32_t chunk, Chunk& t) {
-        const uint32_t row0 = chunk * (uint32_t)kSChunk + (uint32_t)lane * 2;
-        ld_lane(rk0, row0 * KE, t.k0);
-        if constexpr (PAIR) ld_lane(rk1, row0 * KE, t.k1);
-        if constexpr (HAS_V) ld_lane(rv, row0 * VE, t.v);
-        const uint32_t boff = (row0 >> 5) * 4;
-        t.vb = ld_bits(rvn, boff);
-        t.kb = PAIR ? no_bits() : ld_bits(rkn, boff);
-        t.cb = no_bits();
-        if constexpr (MODE == 4) {
-            if (preds.rwide) {
-                ld_lane(rc, row0 * 8, t.c);
-            } else {
-                LaneWords<4> c4;
-                ld_lane(rc, row0 * 4, c4);
-#pragma unroll
-                for (int j = 0; j < kSRows; j++) t.c.w[j] = c4.w[j];
-            }
-            t.cb = ld_bits(rcn, boff);
-        }
-    };
     P1Ring<VT, VV> ring;
-    auto process = [&](uint32_t chunk, const Chunk& t) {
-        const uint32_t row0 = chunk * (uint32_t)kSChunk + (uint32_t)lane * 2;
-        const uint32_t sh = row0 & 31;
-        uint64_t key[kSRows];
-        VV val[kSRows];
-        int ls[kSRows];
-        uint32_t pass = 0, vnl = 0, knl = 0;
-#pragma unroll
-        for (int j = 0; j < kSRows; j++) {
-            const bool vn = t.vb.bit(j, sh);
-            const bool kn = t.kb.bit(j, sh);
-            uint64_t kk;
-            if constexpr (PAIR)
-                kk = (uint64_t)t.k0.w[j] | ((uint64_t)t.k1.w[j] << 32);
-            else
-                kk = (uint64_t)(int64_t)word_elem<KT>(t.k0.w, j);
-            kk = kn ? 0ull : kk;
-            VV v = 0;
-            if constexpr (HAS_V) v = word_elem<VV>(t.v.w, j);
-            int64_t cv = 0;
-            if constexpr (MODE == 4)
-                cv = preds.rwide ? word_elem<int64_t>(t.c.w, j) : (int64_t)word_elem<int32_t>(t.c.w, j);
-            const bool cn = t.cb.bit(j, sh);
-            const bool in_block = row0 + (uint32_t)((j >> 1) * kSPart + (j & 1)) < (uint32_t)n;
-            const bool ok = in_block & row_passes<VT, MODE>(preds, 0u, nullptr, 0, v, vn, cv, cn);
-            key[j] = kk;
-            val[j] = v;
-            pass |= (uint32_t)ok << j;
-            vnl |= (uint32_t)vn << j;
-            knl |= (uint32_t)kn << j;
-        }
+    stream_rows<VT, MODE, KT, kBlock>(kc, vals, vnull, preds, n, [&](const StreamRows<VV>& o) {
         // every row's bucket is read first (a NULL key reads key 0's; the NULL key and the key
         // equal to the empty marker then take their side slots by selection); with no heavy key
         // the table is not read
+        int ls[kSRows];
 #pragma unroll
         for (int j = 0; j < kSRows; j++) {
-            int l = K ? heavy_find(L.lkey, nb, key[j]) : -1;
-            l = key[j] == kEmpty ? H + 1 : l;
-            ls[j] = ((knl >> j) & 1) ? H : l;
+            int l = K ? heavy_find(L.lkey, nb, o.key[j]) : -1;
+            l = o.key[j] == kEmpty ? H + 1 : l;
+            ls[j] = o.knull[j] ? H : l;
         }
 #pragma unroll
         for (int j = 0; j < kSRows; j++)
-            if (((pass >> j) & 1) && ls[j] >= 0) p1_heavy_add<VT>(L, ls[j], val[j], (vnl >> j) & 1);
+            if (o.pass[j] && ls[j] >= 0) p1_heavy_add<VT>(L, ls[j], o.val[j], o.vnull[j]);
         // cold rows with a value go to the ring; a NULL value takes the atomic path
 #pragma unroll
         for (int j = 0; j < kSRows; j++) {
-            const bool vn = (vnl >> j) & 1;
-            const bool cold = ((pass >> j) & 1) & (ls[j] < 0);
-            if (cold && vn) p1_atomic_row<VT>(gp, L.nnew, fields, key[j], hash64(key[j]), val[j], true);
-            ring.push(L, a, gp, fields, cold && !vn, key[j], val[j]);
+            const bool cold = o.pass[j] & (ls[j] < 0);
+            if (cold && o.vnull[j])
+                p1_atomic_row<VT>(gp, L.nnew, fields, o.key[j], hash64(o.key[j]), o.val[j], true);
+            ring.push(L, a, gp, fields, cold && !o.vnull[j], o.key[j], o.val[j]);
         }
-    };
-    // chunks are dealt to the wavefronts of the grid in turn; each wavefront loads its next
-    // chunk before it aggregates the current one (two register sets, used alternately)
-    const uint32_t nchunks = (uint32_t)(((int64_t)n + kSChunk - 1) / kSChunk);
-    const uint32_t stride = gridDim.x * (uint32_t)(kBlock / 64);
-    uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBlock / 64) + (tid >> 6)));
-    Chunk A, B;
-    load(c, A);
-    while (c < nchunks) {
-        load(c + stride, B);
-        process(c, A);
-        c += stride;
-        if (c >= nchunks) break;
-        load(c + stride, A);
-        process(c, B);
-        c += stride;
-    }
+    });
     if (ring.cnt) ring.drain(L, a, gp, fields, ring.cnt);
     p1_end<VTraits<VT>::real>(L, a, gp);
 }
@@ -1711,10 +1501,6 @@ int launch_p1s_m(int mode, TwoPhaseBufs& b, const KeyCols& kc, const void* vals,
     return fail(QK_ERROR, "value range filter without a value column");
 }
 
-// Blocks of at most this many rows take the streaming phase 1 (its loads use 32-bit byte
-// offsets: 8-byte columns and the prefetch past the end stay below 2^31 bytes).
-constexpr int64_t kStreamMaxRows = (int64_t)1 << 27;
-
 // The streaming form for one int64 or int32 key column, or two non-NULL int32 key columns
 // packed into one word, under no WHERE or a folded one; the general form reads any key layout
 // through the key spec and evaluates any WHERE.
@@ -1723,20 +1509,17 @@ int launch_p1_k(int mode, TwoPhaseBufs& b, const KeySpec& ks, const KeyCols& kc,
                 const uint64_t* vnull, const int8_t* mask, const PredSet& ps, uint32_t vpred, int64_t n,
                 uint32_t fields, hipStream_t s) {
     const bool sum_only = (fields & F_SUM) && !(fields & (F_MIN | F_MAX));
-    const bool streamed = (mode == 0 || mode == 3 || mode == 4) && n <= kStreamMaxRows;
-    b.last_form = 1;
-    if (streamed && ks.single && ks.nkeys == 1 && ks.type[0] == QK_LONG) {
+    const bool streamed = stream_keys(ks, kc) && (mode == 0 || mode == 3 || mode == 4) && n <= kStreamMaxRows;
+    b.last_form = streamed ? 1 : 0;
+    if (streamed && !ks.single) return launch_p1s_m<VT, KeyPairI32, kFieldsAny>(mode, b, kc, vals, vnull, ps, n, fields, s);
+    if (streamed && ks.type[0] == QK_LONG) {
         if (sum_only) return launch_p1s_m<VT, int64_t, kFieldsSum>(mode, b, kc, vals, vnull, ps, n, fields, s);
         return launch_p1s_m<VT, int64_t, kFieldsAny>(mode, b, kc, vals, vnull, ps, n, fields, s);
     }
-    if (streamed && ks.single && ks.nkeys == 1 && ks.type[0] == QK_INT) {
+    if (streamed) {
         if (sum_only) return launch_p1s_m<VT, int32_t, kFieldsSum>(mode, b, kc, vals, vnull, ps, n, fields, s);
         return launch_p1s_m<VT, int32_t, kFieldsAny>(mode, b, kc, vals, vnull, ps, n, fields, s);
     }
-    if (streamed && !ks.single && ks.nkeys == 2 && ks.kw == 1 && ks.type[0] == QK_INT && ks.type[1] == QK_INT &&
-        ks.word[0] == 0 && ks.shift[0] == 0 && ks.word[1] == 0 && ks.shift[1] == 32 && !kc.nm[0] && !kc.nm[1])
-        return launch_p1s_m<VT, KeyPairI32, kFieldsAny>(mode, b, kc, vals, vnull, ps, n, fields, s);
-    b.last_form = 0;
     switch (mode) {
     case 0: return launch_p1<VT, 0>(b, ks, kc, vals, vnull, mask, ps, vpred, n, fields, s);
     case 1: return launch_p1<VT, 1>(b, ks, kc, vals, vnull, mask, ps, vpred, n, fields, s);
