@@ -143,6 +143,13 @@ __device__ __forceinline__ T g_load_volatile(const T* p) {
     return *(const volatile __attribute__((address_space(1))) T*)p;
 }
 
+__device__ __forceinline__ uint64_t g_ld_agent(const uint64_t* p) {
+    return __hip_atomic_load(to_g(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void g_st_agent(uint64_t* p, uint64_t v) {
+    __hip_atomic_store(to_g(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 __device__ __forceinline__ uint64_t ld_relaxed(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
