@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 
 #include "../../include/qikkdb_amd.h"
 
@@ -54,8 +55,11 @@ struct Scratch {
     void* ptr = nullptr;
     size_t bytes = 0;
     uint32_t epoch = 0;  // look-back epoch of the last launch on this scratch
+    std::mutex mu;       // for callers that use it over several launches
 };
-int stream_scratch(hipStream_t s, size_t bytes, Scratch** out);
+// kind 0: the look-back kernels' (whose words must hold nothing else); kind 1: a compaction's bits and
+// counts.
+int stream_scratch(hipStream_t s, size_t bytes, Scratch** out, int kind = 0);
 
 // Small pinned host buffer per thread for count read-backs.
 int pinned_host(size_t bytes, void** out);

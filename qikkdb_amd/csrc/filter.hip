@@ -333,6 +333,36 @@ bool fold_column_range(PredSet* ps, uint32_t vpred) {
     return true;
 }
 
+void fold_columns(const PredSet& ps, RangeSet* rs, PredSet* rest) {
+    Fold f[kMaxPreds];
+    rs->n = 0;
+    rest->n = 0;
+    for (int i = 0; i < ps.n; i++) {
+        const qk_predicate& p = ps.p[i];
+        // nothing compares true with a NaN constant, which no interval says
+        if (p.rhs_kind != QK_CONST || !foldable_op(p.op) || (is_real_type(p.rhs_type) && p.rhs_real != p.rhs_real)) {
+            rest->p[rest->n++] = p;
+            continue;
+        }
+        int c = 0;
+        while (c < rs->n && !(rs->c[c].col == p.column && rs->c[c].nm == p.null_mask && rs->c[c].type == p.type)) c++;
+        if (c == rs->n) {
+            rs->c[c].col = p.column;
+            rs->c[c].nm = p.null_mask;
+            rs->c[c].type = p.type;
+            rs->n++;
+        }
+        switch (p.type) {
+        case QK_INT8: fold_typed<int8_t>(p, f[c]); break;
+        case QK_INT: fold_typed<int32_t>(p, f[c]); break;
+        case QK_LONG: fold_typed<int64_t>(p, f[c]); break;
+        case QK_FLOAT: fold_typed<float>(p, f[c]); break;
+        default: fold_typed<double>(p, f[c]); break;
+        }
+    }
+    for (int c = 0; c < rs->n; c++) rs->c[c].vr = range_of(f[c]);
+}
+
 }  // namespace qk
 
 using namespace qk;

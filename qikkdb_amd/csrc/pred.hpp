@@ -125,6 +125,18 @@ struct PredSet {
     int32_t rwide;  // 1: int64, 0: int32
 };
 
+// The comparisons of one column with constants, folded into one interval.
+struct RangeCol {
+    const void* col;
+    const uint64_t* nm;
+    int32_t type;
+    ValueRange vr;
+};
+struct RangeSet {
+    int32_t n;
+    RangeCol c[kMaxPreds];
+};
+
 // The folded range column at row r, widened to int64.
 __device__ __forceinline__ int64_t range_col(const PredSet& ps, int64_t r) {
     return ps.rwide ? __builtin_nontemporal_load((const int64_t*)ps.rcol + r)
@@ -149,5 +161,9 @@ bool fold_value_range(PredSet* ps, uint32_t vpred, int32_t vtype);
 // constant by >, >=, <, <= or ==.  Returns whether it did; the fused kernels then load that
 // column with the rest of a tile and test the interval (a NULL value fails it).
 bool fold_column_range(PredSet* ps, uint32_t vpred);
+
+// Splits a conjunction: the predicates that compare a column with a constant by >, >=, <, <= or ==
+// fold into one interval per column (and null mask), the others stay predicates in `rest`.
+void fold_columns(const PredSet& ps, RangeSet* rs, PredSet* rest);
 
 }  // namespace qk

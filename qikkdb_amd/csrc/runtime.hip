@@ -9,6 +9,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <tuple>
 #include <unordered_map>
 #include <vector>
 
@@ -169,14 +170,14 @@ bool pool_can_allocate(size_t bytes) {
 
 namespace {
 std::mutex g_scratch_mu;
-std::map<std::pair<int, hipStream_t>, Scratch*> g_scratch;
+std::map<std::tuple<int, hipStream_t, int>, Scratch*> g_scratch;
 }  // namespace
 
-int stream_scratch(hipStream_t s, size_t bytes, Scratch** out) {
+int stream_scratch(hipStream_t s, size_t bytes, Scratch** out, int kind) {
     int dev = 0;
     QK_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(g_scratch_mu);
-    Scratch*& sc = g_scratch[{dev, s}];
+    Scratch*& sc = g_scratch[{dev, s, kind}];
     if (!sc) sc = new Scratch();
     if (sc->bytes < bytes) {
         size_t nb = 1 << 16;
