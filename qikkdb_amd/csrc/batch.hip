@@ -23,6 +23,11 @@
 // unit whose rows do not fit takes the atomic path.  Rows per query are estimated by sampling
 // before the run.
 //
+// A batch that reads its rows many times over first copies the tiles it touches in ts order, chunk by
+// chunk (k_batch_sort): the rows of 4096 grouped into 64 ranges of ts, with the key's a * b_range + b
+// computed.  A query then reads from every chunk only the contiguous rows of the ranges its window
+// meets, and compares ts only in the window's two outermost ranges.  The copy is made by every run.
+//
 // Results are dense arrays indexed by out_i + key.  MIN/MAX are kept in an order-preserving
 // unsigned encoding during the run and decoded at its end.
 #include <algorithm>
@@ -44,6 +49,17 @@ constexpr int kXcds = 8;             // dies of the device, each with its own L2
 constexpr int kCtrStride = 16;       // counters per wave: kXcds unit lists, pass-2 units, pool top
 constexpr int kCtrPass2 = kXcds;
 constexpr int kCtrPool = kXcds + 1;
+// The ts-ordered copy: rows per chunk, ranges of ts per chunk (one boundary per lane of a wavefront in
+// the search), start offsets kept per chunk (padded), and the bytes of a copied row.
+constexpr int kSortRows = 4096;
+constexpr int kRanges = 64;
+constexpr int kRangeStride = kRanges + 2;
+constexpr int kSortThreads = 512;
+constexpr int64_t kSortRowBytes = 20;
+constexpr int64_t kSortMaxBytes = (int64_t)24 << 30;
+// A batch sorts when its queries read the rows of its tiles at least this many times: the copy moves
+// 44 bytes per row, about four reads' worth of what it saves.
+constexpr int64_t kSortMinReads = 6;
 
 struct BQuery {
     int64_t row0, rows;   // table rows of the query
@@ -59,7 +75,7 @@ struct BQuery {
     int32_t chunks;       // large: key chunks; 0 for a small query
     int32_t cbits;        // large: chunk = key >> cbits
     int32_t index;        // position in the caller's list
-    int32_t pad;
+    uint32_t magic32;     // floor(2^32 / key_mod), at most 2^32 - 1
 };
 
 struct BUnit {
@@ -78,6 +94,7 @@ struct BHeader {
     int64_t out_total;
     int64_t scratch_cap;  // rows
     int64_t nunits;
+    int64_t sort_tile0, sort_tiles;  // tiles copied in ts order
 };
 
 struct BArgs {
@@ -105,6 +122,17 @@ struct BArgs {
     unsigned long long* sum;
     unsigned long long* mn;
     unsigned long long* mx;
+    // the ts-ordered copy (null: this batch reads the columns): key numbers a * b_range + b, values, ts;
+    // per chunk the start of each range; per block the ranges' boundaries; per tile whether a key number
+    // does not fit 32 bits (such tiles are read from the columns)
+    int64_t rows;
+    int32_t block_rows;
+    uint32_t* ox;
+    int64_t* ov;
+    int64_t* ots;
+    uint16_t* ostart;
+    const int64_t* bounds;
+    uint32_t* owide;
 };
 
 // x mod d for 0 <= x < 2^32 and 1 <= d < 2^32 (Lemire, Kaser and Kurz, "Faster remainder by
@@ -115,6 +143,12 @@ __device__ __forceinline__ uint32_t key_of(int32_t a, int32_t b, int32_t b_range
     int64_t r = x % q.mod;
     if (r < 0) r += q.mod;
     return (uint32_t)r;
+}
+
+// x mod d with q = floor(x * floor(2^32 / d) / 2^32), which is the quotient or one less.
+__device__ __forceinline__ uint32_t mod32(uint32_t x, const BQuery& q) {
+    const uint32_t r = x - __umulhi(x, q.magic32) * (uint32_t)q.mod;
+    return r >= (uint32_t)q.mod ? r - (uint32_t)q.mod : r;
 }
 
 // A value every lane holds the same copy of, moved to scalar registers so that branches on it
@@ -175,6 +209,8 @@ __global__ void __launch_bounds__(256) k_batch_init(BArgs p) {
         p.comp[i] = 0;
     }
     for (uint64_t i = i0; i < (uint64_t)kCtrStride * h.nwaves; i += stride) p.ctr[i] = 0;
+    if (p.ox)
+        for (uint64_t i = i0; i < (uint64_t)h.sort_tiles; i += stride) p.owide[h.sort_tile0 + i] = 0;
     if (i0 == 0) *p.t0 = wall_clock64();
 }
 
@@ -201,6 +237,144 @@ __global__ void __launch_bounds__(256) k_batch_sample_ts(const int64_t* __restri
     }
 }
 
+// The ts-ordered copy of the batch's tiles, one chunk of kSortRows rows per workgroup and turn: each row's
+// range by a binary search over the block's boundaries in LDS, its place by a counter per range, the
+// rows permuted in LDS and written out in order.
+__global__ void __launch_bounds__(kSortThreads) k_batch_sort(BArgs p) {
+    __shared__ int64_t s_bound[kRanges];
+    __shared__ uint32_t s_cnt[kRanges];
+    __shared__ int64_t s_v[kSortRows];  // values, then key numbers: two workgroups fit a CU
+    __shared__ int64_t s_t[kSortRows];
+    uint32_t* s_x = (uint32_t*)s_v;
+    constexpr int kPer = kSortRows / kSortThreads;
+    const BHeader h = *p.hdr;
+    const int tid = threadIdx.x;
+    const int64_t per_tile = p.tile_rows / kSortRows;
+    const int64_t c_end = min((h.sort_tile0 + h.sort_tiles) * per_tile, (p.rows + kSortRows - 1) / kSortRows);
+    for (int64_t c = h.sort_tile0 * per_tile + blockIdx.x; c < c_end; c += gridDim.x) {
+        const int64_t row0 = c * kSortRows;
+        const int n = (int)min((int64_t)kSortRows, p.rows - row0);
+        const int64_t tile = c / per_tile;
+        const int64_t blk = tile * p.tile_rows / p.block_rows;
+        int64_t t[kPer], v[kPer];
+        int32_t a[kPer], b[kPer];
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int64_t r = row0 + min(k * kSortThreads + tid, n - 1);
+            t[k] = __builtin_nontemporal_load(p.ts + r);
+            a[k] = __builtin_nontemporal_load(p.a + r);
+            b[k] = __builtin_nontemporal_load(p.b + r);
+            v[k] = __builtin_nontemporal_load(p.v + r);
+        }
+        if (tid < kRanges) {
+            s_bound[tid] = tid < kRanges - 1 ? p.bounds[blk * kRanges + tid] : INT64_MAX;
+            s_cnt[tid] = 0;
+        }
+        __syncthreads();
+        uint32_t place[kPer];  // range, then rank in it
+        bool wide = false;
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            uint32_t g = 0;  // boundaries <= ts among the first kRanges - 1
+#pragma unroll
+            for (int d = kRanges / 2; d >= 1; d >>= 1) g += s_bound[g + d - 1] <= t[k] ? d : 0;
+            place[k] = g << 16;
+            if (k * kSortThreads + tid < n) {
+                place[k] |= atomicAdd(&s_cnt[g], 1u);
+                wide |= (uint64_t)((int64_t)a[k] * p.b_range + b[k]) >> 32 != 0;
+            }
+        }
+        __syncthreads();
+        if (tid < 64) {
+            const uint32_t mine = s_cnt[tid];
+            const uint32_t at = (uint32_t)wave_incl_scan((int32_t)mine, tid) - mine;
+            s_cnt[tid] = at;
+            p.ostart[c * kRangeStride + tid] = (uint16_t)at;
+            if (tid == 63) p.ostart[c * kRangeStride + kRanges] = (uint16_t)n;
+        }
+        if (__any(wide) && (tid & 63) == 0) atomicOr(p.owide + tile, 1u);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            place[k] = s_cnt[place[k] >> 16] + (place[k] & 0xffffu);
+            if (k * kSortThreads + tid >= n) continue;
+            s_v[place[k]] = v[k];
+            s_t[place[k]] = t[k];
+        }
+        __syncthreads();
+        for (int i = tid; i < n; i += kSortThreads) {
+            p.ov[row0 + i] = s_v[i];
+            p.ots[row0 + i] = s_t[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kPer; k++)
+            if (k * kSortThreads + tid < n) s_x[place[k]] = (uint32_t)((int64_t)a[k] * p.b_range + b[k]);
+        __syncthreads();
+        for (int i = tid; i < n; i += kSortThreads) p.ox[row0 + i] = s_x[i];
+        __syncthreads();
+    }
+}
+
+// Hands every row of a tile that lies in [r_begin, r_end) and passes the query's window to
+// f(key, value, pass), from the ts-ordered copy (f is called by all 64 lanes).  A wavefront takes whole
+// chunks; a chunk the query covers in part (its ends, or a tile of wide key numbers) is read from
+// the columns.  Two sweeps over the same unit see the same rows.
+template <bool NEED_V, typename F>
+__device__ __forceinline__ void ordered_rows(const BArgs& p, const BQuery& Q, int64_t tile, int64_t r_begin,
+                                             int64_t r_end, F&& f) {
+    if (Q.ts_hi <= Q.ts_lo) return;
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwv = blockDim.x >> 6;
+    // ranges of the window's ends: boundaries <= the end, one boundary per lane
+    const int64_t blk = tile * p.tile_rows / p.block_rows;
+    const int64_t bound = lane < kRanges - 1 ? p.bounds[blk * kRanges + lane] : INT64_MAX;
+    const int g_lo = __popcll(__ballot(lane < kRanges - 1 && bound <= Q.ts_lo));
+    const int g_hi = __popcll(__ballot(lane < kRanges - 1 && bound <= Q.ts_hi));
+    const bool wide = __builtin_amdgcn_readfirstlane((int)p.owide[tile]) != 0;
+    const int64_t c0 = tile * p.tile_rows / kSortRows;
+    const int nchunks = p.tile_rows / kSortRows;
+    for (int i = wid; i < nchunks; i += nwv) {
+        const int64_t row0 = (c0 + i) * kSortRows;
+        const int64_t row1 = min(row0 + kSortRows, p.rows);
+        if (row0 >= r_end || row1 <= r_begin) continue;
+        if (wide || row0 < r_begin || row1 > r_end) {
+            const int64_t lo = max(row0, r_begin), hi = min(row1, r_end);
+            for (int64_t r0 = lo; r0 < hi; r0 += 64) {
+                const int64_t r = min(r0 + lane, hi - 1);
+                const int64_t t = p.ts[r];
+                const uint32_t key = key_of(p.a[r], p.b[r], p.b_range, Q);
+                const int64_t v = NEED_V ? p.v[r] : 0;
+                f(key, v, (r0 + lane < hi) & (t >= Q.ts_lo) & (t < Q.ts_hi));
+            }
+            continue;
+        }
+        const uint16_t* st = p.ostart + (c0 + i) * kRangeStride;
+        const int lo0 = __builtin_amdgcn_readfirstlane((int)st[g_lo]);
+        const int lo1 = __builtin_amdgcn_readfirstlane((int)st[g_lo + 1]);
+        const int hi0 = __builtin_amdgcn_readfirstlane((int)st[g_hi]);
+        const int hi1 = __builtin_amdgcn_readfirstlane((int)st[g_hi + 1]);
+        constexpr int kU = 4;
+        for (int j0 = lo0; j0 < hi1; j0 += 64 * kU) {
+            uint32_t x[kU];
+            int64_t v[kU], t[kU];
+            bool test[kU];
+#pragma unroll
+            for (int u = 0; u < kU; u++) {
+                const int j = min(j0 + u * 64 + lane, hi1 - 1);
+                x[u] = p.ox[row0 + j];
+                v[u] = NEED_V ? p.ov[row0 + j] : 0;
+                test[u] = (j < lo1) | (j >= hi0);
+                t[u] = Q.ts_lo;
+                if (test[u]) t[u] = p.ots[row0 + j];
+            }
+#pragma unroll
+            for (int u = 0; u < kU; u++)
+                f(mod32(x[u], Q), v[u], (j0 + u * 64 + lane < hi1) & (t[u] >= Q.ts_lo) & (t[u] < Q.ts_hi));
+        }
+    }
+}
+
 // Claims the next pass-1 unit of a wave: first from the list of this workgroup's die (units
 // of one tile share that die's L2), then from the other lists once it is empty.  -1 when
 // every list is empty.  `xi` is the caller's position in that order.
@@ -218,6 +392,8 @@ __device__ __forceinline__ int64_t claim_unit(const BArgs& p, const BWave& W, in
     return -1;
 }
 
+// ORDERED: rows come from the ts-ordered copy.
+template <bool ORDERED>
 __global__ void __launch_bounds__(kBThreads) k_batch_pass1(BArgs p, int32_t wave) {
     extern __shared__ __align__(16) uint64_t lds[];
     __shared__ int64_t s_unit, s_base;
@@ -260,6 +436,16 @@ __global__ void __launch_bounds__(kBThreads) k_batch_pass1(BArgs p, int32_t wave
                 lcnt[g] = 0;
             }
             __syncthreads();
+            if constexpr (ORDERED) {
+                ordered_rows<true>(p, Q, tile, r_begin, r_end, [&](uint32_t key, int64_t v, bool pass) {
+                    if (!pass) return;
+                    const uint64_t e = enc_i64(v);
+                    atomicAdd(&lcnt[key], 1u);
+                    atomicAdd((unsigned long long*)&lsum[key], (unsigned long long)v);
+                    atomicMin((unsigned long long*)&lmn[key], (unsigned long long)e);
+                    atomicMax((unsigned long long*)&lmx[key], (unsigned long long)e);
+                });
+            } else
             // every column of a step is loaded at once (one wait per step); most of these
             // lines are read by other queries of the same tile anyway
             for (int64_t base = r_begin; base < r_end; base += (int64_t)bd * kBRows) {
@@ -301,6 +487,11 @@ __global__ void __launch_bounds__(kBThreads) k_batch_pass1(BArgs p, int32_t wave
             for (int c = tid; c < nch; c += bd) hist[c] = 0;
             __syncthreads();
             int word = wid;
+            if constexpr (ORDERED) {
+                ordered_rows<false>(p, Q, tile, r_begin, r_end, [&](uint32_t key, int64_t, bool pass) {
+                    if (pass) atomicAdd(&hist[key >> cbits], 1u);
+                });
+            } else
             for (int64_t base = r_begin; base < r_end; base += (int64_t)bd * kBRows) {
                 int64_t tsv[kBRows];
                 int32_t av[kBRows], bv[kBRows];
@@ -344,6 +535,19 @@ __global__ void __launch_bounds__(kBThreads) k_batch_pass1(BArgs p, int32_t wave
             __syncthreads();
             const int64_t sbase = uniform64(s_base);
             word = wid;
+            if constexpr (ORDERED) {
+                ordered_rows<true>(p, Q, tile, r_begin, r_end, [&](uint32_t key, int64_t val, bool pass) {
+                    if (!pass) return;
+                    if (sbase >= 0) {
+                        const uint32_t at = atomicAdd(&cur[key >> cbits], 1u);
+                        p.sk[sbase + at] = key;
+                        p.sv[sbase + at] = val;
+                    } else {
+                        const uint64_t e = enc_i64(val);
+                        add_global(p, Q.out + key, 1u, val, e, e);
+                    }
+                });
+            } else
             for (int64_t base = r_begin; base < r_end; base += (int64_t)bd * kBRows) {
                 int32_t av[kBRows], bv[kBRows];
                 int64_t vv[kBRows];
@@ -469,6 +673,10 @@ __global__ void __launch_bounds__(256) k_key_column(const int32_t* __restrict__ 
         out[i] = key_of(a[i], b[i], b_range, q);
 }
 
+uint32_t magic32_of(int32_t mod) {
+    return (uint32_t)std::min<uint64_t>(((uint64_t)1 << 32) / (uint64_t)(uint32_t)mod, 0xffffffffull);
+}
+
 uint64_t magic_of(int32_t mod) { return ~0ull / (uint64_t)(uint32_t)mod + 1; }
 
 // Widest key chunk of the two-pass path: the largest power of two <= max(lds_groups, 1024).
@@ -541,6 +749,15 @@ struct qk_batch_s {
     std::vector<int64_t> samples;
     int32_t per_block = 0;
     int32_t last_nq = 0;
+    // the ts-ordered copy of the table (filled by each run that uses it) and the ranges' boundaries
+    bool order_ok = true;  // the owner allows it (batch_allow_order)
+    uint32_t* ox = nullptr;
+    int64_t *ov = nullptr, *ots = nullptr;
+    uint16_t* ostart = nullptr;
+    uint32_t* owide = nullptr;
+    int64_t order_tiles = 0;  // tiles owide has room for
+    int64_t* bounds = nullptr;
+    int64_t bound_blocks = 0;
     // captured graph of init -> waves -> finalize, valid while the launch arguments match
     hipGraphExec_t graph = nullptr;
     int32_t graph_waves = -1;
@@ -585,8 +802,23 @@ void free_plan(qk_batch_s* b) {
     b->q_cap = b->wave_cap = 0;
 }
 
+void free_order(qk_batch_s* b) {
+    void* ptrs[] = {b->ox, b->ov, b->ots, b->ostart};
+    for (void* p : ptrs)
+        if (p) pool_free(p);
+    b->ox = nullptr;
+    b->ov = b->ots = nullptr;
+    b->ostart = nullptr;
+}
+
 void free_buffers(qk_batch_s* b) {
     free_plan(b);
+    free_order(b);
+    if (b->owide) pool_free(b->owide);
+    if (b->bounds) pool_free(b->bounds);
+    b->owide = nullptr;
+    b->bounds = nullptr;
+    b->order_tiles = b->bound_blocks = 0;
     void* ptrs[] = {b->units, b->desc, b->segb, b->sk, b->sv, b->cnt, b->sum, b->mn, b->mx};
     for (void* p : ptrs)
         if (p) pool_free(p);
@@ -604,8 +836,9 @@ void free_buffers(qk_batch_s* b) {
     free_graph(b);
 }
 
-BArgs args_of(const qk_batch_s* b) {
+BArgs args_of(const qk_batch_s* b, bool ordered) {
     BArgs p;
+    memset((void*)&p, 0, sizeof p);  // padding too: arguments are compared bytewise
     p.a = b->cols.a;
     p.b = b->cols.b;
     p.ts = b->cols.ts;
@@ -630,16 +863,37 @@ BArgs args_of(const qk_batch_s* b) {
     p.sum = b->res[1];
     p.mn = b->res[2];
     p.mx = b->res[3];
+    p.rows = b->cols.rows;
+    p.block_rows = b->cols.block_rows;
+    p.ox = nullptr;
+    p.ov = p.ots = nullptr;
+    p.ostart = nullptr;
+    p.bounds = nullptr;
+    p.owide = nullptr;
+    if (ordered) {
+        p.ox = b->ox;
+        p.ov = b->ov;
+        p.ots = b->ots;
+        p.ostart = b->ostart;
+        p.bounds = b->bounds;
+        p.owide = b->owide;
+    }
     return p;
 }
 
-int launch_all(qk_batch_s* b, int32_t nwaves, hipStream_t s) {
-    const BArgs p = args_of(b);
+int launch_all(qk_batch_s* b, int32_t nwaves, bool ordered, hipStream_t s) {
+    const BArgs p = args_of(b, ordered);
     const int cus = device_info().cus;
     k_batch_init<<<cus * 8, 256, 0, s>>>(p);
     QK_HIP(hipGetLastError());
+    if (ordered) {
+        k_batch_sort<<<cus * 2, kSortThreads, 0, s>>>(p);
+        QK_HIP(hipGetLastError());
+    }
     for (int32_t w = 0; w < nwaves; w++) {
-        k_batch_pass1<<<cus * b->tune.wgs_per_cu, kBThreads, pass1_lds_bytes(b->tune), s>>>(p, w);
+        const unsigned grid = (unsigned)(cus * b->tune.wgs_per_cu);
+        if (ordered) k_batch_pass1<true><<<grid, kBThreads, pass1_lds_bytes(b->tune), s>>>(p, w);
+        else k_batch_pass1<false><<<grid, kBThreads, pass1_lds_bytes(b->tune), s>>>(p, w);
         QK_HIP(hipGetLastError());
         k_batch_pass2<<<cus * b->tune.wgs_per_cu, kBThreads, pass2_lds_bytes(b->tune), s>>>(p, w);
         QK_HIP(hipGetLastError());
@@ -650,7 +904,7 @@ int launch_all(qk_batch_s* b, int32_t nwaves, hipStream_t s) {
 }
 
 // Capture init -> waves -> finalize once for the current buffers, tuning and wave count.
-void build_graph(qk_batch_s* b, int32_t nwaves) {
+void build_graph(qk_batch_s* b, int32_t nwaves, bool ordered) {
     free_graph(b);
     hipStream_t cs = nullptr;
     if (hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) != hipSuccess) {
@@ -660,7 +914,7 @@ void build_graph(qk_batch_s* b, int32_t nwaves) {
     hipGraph_t g = nullptr;
     bool ok = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) == hipSuccess;
     if (ok) {
-        const int lst = launch_all(b, nwaves, cs);
+        const int lst = launch_all(b, nwaves, ordered, cs);
         const hipError_t e = hipStreamEndCapture(cs, &g);
         ok = lst == QK_SUCCESS && e == hipSuccess;
     }
@@ -726,6 +980,35 @@ int ensure_units(qk_batch_s* b, int64_t n) {
     return QK_SUCCESS;
 }
 
+// The ts-ordered copy's memory (for the whole table); false when the owner does not allow it, the table is
+// too large for it or there is no memory left: the batch then reads the columns.
+bool ensure_order(qk_batch_s* b) {
+    const int64_t rows = b->cols.rows;
+    if (!b->order_ok || !b->bounds || rows < kSortRows || rows > kSortMaxBytes / kSortRowBytes) return false;
+    const int64_t chunks = (rows + kSortRows - 1) / kSortRows;
+    const int64_t tiles = (rows + b->tune.tile_rows - 1) / b->tune.tile_rows;
+    if (!b->ox) {
+        free_graph(b);
+        int st = pool_alloc((void**)&b->ox, (size_t)rows * 4);
+        if (st == QK_SUCCESS) st = pool_alloc((void**)&b->ov, (size_t)rows * 8);
+        if (st == QK_SUCCESS) st = pool_alloc((void**)&b->ots, (size_t)rows * 8);
+        if (st == QK_SUCCESS) st = pool_alloc((void**)&b->ostart, (size_t)chunks * kRangeStride * 2);
+        if (st != QK_SUCCESS) {
+            free_order(b);
+            return false;
+        }
+    }
+    if (b->order_tiles < tiles) {
+        free_graph(b);
+        if (b->owide) pool_free(b->owide);
+        b->owide = nullptr;
+        b->order_tiles = 0;
+        if (pool_alloc((void**)&b->owide, (size_t)tiles * 4) != QK_SUCCESS) return false;
+        b->order_tiles = tiles;
+    }
+    return true;
+}
+
 // Units of queries [q_begin, q_end) of the plan, appended at out[*n] as kXcds lists: list x
 // holds the tiles t with t mod kXcds == x, tile by tile (the queries of a tile in plan order).
 void list_units(const std::vector<BQuery>& bq, BWave* w, BUnit* out, int64_t* n) {
@@ -779,6 +1062,19 @@ int take_samples(qk_batch_s* b) {
     if (e != hipSuccess) return fail(QK_RUNTIME_ERROR, "qk_batch: sampling ts: %s", hipGetErrorString(e));
     for (int64_t blk = 0; blk < nblocks; blk++)
         std::sort(b->samples.begin() + blk * per, b->samples.begin() + (blk + 1) * per);
+    // each block's boundaries of kRanges ranges of ts: quantiles of its samples
+    std::vector<int64_t> bounds((size_t)(nblocks * kRanges), INT64_MAX);
+    for (int64_t blk = 0; blk < nblocks; blk++)
+        for (int64_t g = 1; g < kRanges; g++)
+            bounds[(size_t)(blk * kRanges + g - 1)] = b->samples[(size_t)(blk * per + g * per / kRanges)];
+    if (b->bound_blocks < nblocks) {
+        if (b->bounds) pool_free(b->bounds);
+        b->bounds = nullptr;
+        b->bound_blocks = 0;
+        if (pool_alloc((void**)&b->bounds, bounds.size() * 8) != QK_SUCCESS) return QK_SUCCESS;
+        b->bound_blocks = nblocks;
+    }
+    QK_HIP(hipMemcpy(b->bounds, bounds.data(), bounds.size() * 8, hipMemcpyHostToDevice));
     return QK_SUCCESS;
 }
 
@@ -843,6 +1139,7 @@ int run_batch(qk_batch_s* b, int32_t nq, const qk_batch_query* q, hipStream_t s,
         d.out = b->offsets[(size_t)i];
         d.mod = x.key_mod;
         d.magic = magic_of(x.key_mod);
+        d.magic32 = magic32_of(x.key_mod);
         d.index = i;
         nlarge += x.key_mod > t.lds_groups;
     }
@@ -940,18 +1237,31 @@ int run_batch(qk_batch_s* b, int32_t nq, const qk_batch_query* q, hipStream_t s,
     hd.out_total = out;
     hd.scratch_cap = nlarge ? pool : 0;
     hd.nunits = nunits;
+    // the tiles the batch touches, and whether it reads their rows often enough to sort them
+    int64_t t_lo = INT64_MAX, t_hi = 0, reads = 0;
+    for (const BQuery& d : bq) {
+        t_lo = std::min(t_lo, d.tile0);
+        t_hi = std::max(t_hi, d.tile0 + d.units);
+        reads += d.rows;
+    }
+    bool ordered = t_lo < t_hi && reads >= kSortMinReads * (t_hi - t_lo) * T;
+    if (ordered) ordered = ensure_order(b);
+    if (ordered) {
+        hd.sort_tile0 = t_lo;
+        hd.sort_tiles = t_hi - t_lo;
+    }
     BQuery* host_q = (BQuery*)((char*)b->host_plan + sizeof(BHeader) + sizeof(BWave) * (size_t)b->wave_cap);
     memcpy(b->host_plan, &hd, sizeof hd);
     memcpy((char*)b->host_plan + sizeof hd, waves.data(), sizeof(BWave) * (size_t)nw);
     if (nq) memcpy(host_q, bq.data(), sizeof(BQuery) * (size_t)nq);
-    const BArgs p = args_of(b);
+    const BArgs p = args_of(b, ordered);
     QK_HIP(hipMemcpyAsync(b->plan, b->host_plan, sizeof hd + sizeof(BWave) * (size_t)nw, hipMemcpyHostToDevice, s));
     if (nq) QK_HIP(hipMemcpyAsync((void*)p.q, host_q, sizeof(BQuery) * (size_t)nq, hipMemcpyHostToDevice, s));
     if (nunits) QK_HIP(hipMemcpyAsync(b->units, b->host_units, sizeof(BUnit) * (size_t)nunits, hipMemcpyHostToDevice, s));
     b->last_nq = nq;
     if (t.use_graph) {
         if (b->graph_waves != nw || memcmp(&p, &b->graph_args, sizeof p) != 0) {
-            build_graph(b, nw);
+            build_graph(b, nw, ordered);
             b->graph_args = p;
         }
         if (b->graph_waves == nw) {
@@ -959,10 +1269,17 @@ int run_batch(qk_batch_s* b, int32_t nq, const qk_batch_query* q, hipStream_t s,
             return QK_SUCCESS;
         }
     }
-    return launch_all(b, nw, s);
+    return launch_all(b, nw, ordered, s);
 }
 
 }  // namespace
+
+void batch_allow_order(qk_batch b, bool allow) { b->order_ok = allow; }
+int64_t batch_order_bytes(const qk_batch_columns& c) {
+    if (c.rows < kSortRows || c.rows > kSortMaxBytes / kSortRowBytes) return 0;
+    return c.rows * kSortRowBytes + c.rows / kSortRows * (kRangeStride * 2 + 4) + (8 << 20);
+}
+
 }  // namespace qk
 
 extern "C" {
@@ -984,6 +1301,7 @@ int qk_batch_create(qk_batch* out, const qk_batch_columns* cols) {
     b->tune.scratch_rows = 0;
     const int st = take_samples(b);
     if (st != QK_SUCCESS) {
+        free_buffers(b);
         delete b;
         return st;
     }

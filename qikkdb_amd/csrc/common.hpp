@@ -64,6 +64,11 @@ int stream_scratch(hipStream_t s, size_t bytes, Scratch** out, int kind = 0);
 // Small pinned host buffer per thread for count read-backs.
 int pinned_host(size_t bytes, void** out);
 
+// Whether a batch engine may keep a ts-ordered copy of its table (batch.hip; on by default), and the
+// device memory the copy takes (0: the table has none).
+void batch_allow_order(qk_batch b, bool allow);
+int64_t batch_order_bytes(const qk_batch_columns& c);
+
 // Resolves and clears the current device's fixed scratch of qk_prefix_sum_noalloc (once per
 // device; called by qk_init).
 int prefix_noalloc_setup();

@@ -353,6 +353,7 @@ int qk_serve_create(qk_serve* out, const qk_batch_columns* cols, const qk_serve_
     }
     if (c.engines < 1 || c.engines > 8 || c.max_batch < 1 || c.memory_cap < 1 || c.wait_ms < 0)
         return qk::fail(QK_ERROR, "qk_serve_create: engines 1..8, max_batch >= 1, memory_cap >= 1, wait_ms >= 0");
+    bool order = true;  // the engines may keep ts-ordered copies of the table
     {
         // Each engine keeps its row pool (12 bytes per pooled row, grown to the largest batch it
         // ran) beside the bytes the cap admits, so the engines share what the device has free
@@ -364,12 +365,16 @@ int qk_serve_create(qk_serve* out, const qk_batch_columns* cols, const qk_serve_
             return qk::fail(QK_RUNTIME_ERROR, "qk_serve_create: hipMemGetInfo failed");
         }
         const int64_t spare = (int64_t)free_b - c.memory_cap;
-        const int64_t rows = spare > 0 ? spare / 10 * 9 / c.engines / 12 : 0;
+        int64_t rows = spare > 0 ? spare / 10 * 9 / c.engines / 12 : 0;
         if (rows < ((int64_t)1 << 20))
             return qk::fail(QK_OUT_OF_MEMORY,
                             "qk_serve_create: a memory cap of %lld bytes leaves %lld of the %zu free bytes for "
                             "the row pools of %d engines", (long long)c.memory_cap, (long long)std::max<int64_t>(spare, 0),
                             free_b, c.engines);
+        // the copies share that memory with the pools, and have at most half of it
+        const int64_t copy_rows = qk::batch_order_bytes(*cols) / 12;
+        order = copy_rows <= rows / 2;
+        if (order) rows -= copy_rows;
         if (c.tuning.scratch_rows <= 0 || c.tuning.scratch_rows > rows) c.tuning.scratch_rows = rows;
     }
     qk_serve_s* s = new (std::nothrow) qk_serve_s();
@@ -382,6 +387,7 @@ int qk_serve_create(qk_serve* out, const qk_batch_columns* cols, const qk_serve_
     int st = QK_SUCCESS;
     for (Engine& e : s->eng) {
         st = qk_batch_create(&e.b, cols);
+        if (st == QK_SUCCESS) qk::batch_allow_order(e.b, order);
         if (st == QK_SUCCESS) st = qk_batch_set_tuning(e.b, &c.tuning);
         if (st == QK_SUCCESS && (hipStreamCreateWithFlags(&e.s, hipStreamNonBlocking) != hipSuccess ||
                                  hipEventCreateWithFlags(&e.done, hipEventDisableTiming) != hipSuccess)) {
