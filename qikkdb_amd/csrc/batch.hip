@@ -429,21 +429,30 @@ __global__ void __launch_bounds__(kBThreads) k_batch_pass1(BArgs p, int32_t wave
             uint64_t* lmn = (uint64_t*)(lsum + G);
             uint64_t* lmx = lmn + G;
             uint32_t* lcnt = (uint32_t*)(lmx + G);
-            for (int g = tid; g < Q.mod; g += bd) {
+            // few groups are kept in up to 32 copies, a lane adding to the copy of its number, as far as
+            // they fit: the lanes would otherwise queue at the same LDS words (a sixth of the mix has
+            // under ten groups)
+            int rb = 0;
+            while (rb < 5 && ((int64_t)Q.mod << (rb + 1)) <= G) rb++;
+            const uint32_t copy = (uint32_t)tid & ((1u << rb) - 1);
+            for (int g = tid; g < Q.mod << rb; g += bd) {
                 lsum[g] = 0;
                 lmn[g] = ~0ull;
                 lmx[g] = 0;
                 lcnt[g] = 0;
             }
             __syncthreads();
+            auto add = [&](uint32_t key, int64_t v) {
+                const uint32_t g = (key << rb) | copy;
+                const uint64_t e = enc_i64(v);
+                atomicAdd(&lcnt[g], 1u);
+                atomicAdd((unsigned long long*)&lsum[g], (unsigned long long)v);
+                atomicMin((unsigned long long*)&lmn[g], (unsigned long long)e);
+                atomicMax((unsigned long long*)&lmx[g], (unsigned long long)e);
+            };
             if constexpr (ORDERED) {
                 ordered_rows<true>(p, Q, tile, r_begin, r_end, [&](uint32_t key, int64_t v, bool pass) {
-                    if (!pass) return;
-                    const uint64_t e = enc_i64(v);
-                    atomicAdd(&lcnt[key], 1u);
-                    atomicAdd((unsigned long long*)&lsum[key], (unsigned long long)v);
-                    atomicMin((unsigned long long*)&lmn[key], (unsigned long long)e);
-                    atomicMax((unsigned long long*)&lmx[key], (unsigned long long)e);
+                    if (pass) add(key, v);
                 });
             } else
             // every column of a step is loaded at once (one wait per step); most of these
@@ -463,18 +472,23 @@ __global__ void __launch_bounds__(kBThreads) k_batch_pass1(BArgs p, int32_t wave
                 for (int k = 0; k < kBRows; k++) {
                     const int64_t r = base + (int64_t)k * bd + tid;
                     const bool pass = (r < r_end) & (tsv[k] >= Q.ts_lo) & (tsv[k] < Q.ts_hi);
-                    if (!pass) continue;
-                    const uint32_t key = key_of(av[k], bv[k], p.b_range, Q);
-                    const uint64_t e = enc_i64(vv[k]);
-                    atomicAdd(&lcnt[key], 1u);
-                    atomicAdd((unsigned long long*)&lsum[key], (unsigned long long)vv[k]);
-                    atomicMin((unsigned long long*)&lmn[key], (unsigned long long)e);
-                    atomicMax((unsigned long long*)&lmx[key], (unsigned long long)e);
+                    if (pass) add(key_of(av[k], bv[k], p.b_range, Q), vv[k]);
                 }
             }
             __syncthreads();
-            for (int g = tid; g < Q.mod; g += bd)
-                if (lcnt[g]) add_global(p, Q.out + g, lcnt[g], lsum[g], lmn[g], lmx[g]);
+            for (int g = tid; g < Q.mod; g += bd) {
+                uint32_t c = 0;
+                int64_t sm = 0;
+                uint64_t mn = ~0ull, mx = 0;
+                for (int i = 0; i < 1 << rb; i++) {  // from the thread's own copy on: other banks than its neighbours
+                    const int at = (g << rb) | ((i + tid) & ((1 << rb) - 1));
+                    c += lcnt[at];
+                    sm += lsum[at];
+                    mn = min(mn, lmn[at]);
+                    mx = max(mx, lmx[at]);
+                }
+                if (c) add_global(p, Q.out + g, c, sm, mn, mx);
+            }
         } else {
             // large query, pass 1: rows per chunk, one slice of the pool, rows written by chunk.
             // The first sweep keeps one pass bit per row in LDS (a wavefront ballot per 64
