@@ -97,6 +97,17 @@ struct BHeader {
     int64_t sort_tile0, sort_tiles;  // tiles copied in ts order
 };
 
+// A row in the scratch pool: its key and value in one 12-byte record, so that a row costs one store.
+// The stores go to the chunks' places, a line of its own per lane, and bind the first pass by their
+// number (256 queries over 128M rows, 1.1 G pooled rows: 9.0 ms with keys and values apart, 7.6 ms so; the
+// second pass, which reads them, 2.7 -> 2.9 ms).
+struct alignas(4) PoolRow {
+    uint32_t w[3];
+};
+__device__ __forceinline__ PoolRow pool_row(uint32_t key, int64_t v) {
+    return {{key, (uint32_t)v, (uint32_t)((uint64_t)v >> 32)}};
+}
+
 struct BArgs {
     const int32_t* a;
     const int32_t* b;
@@ -116,8 +127,7 @@ struct BArgs {
     unsigned long long* comp;   // [nq, caller order] completion clock
     int32_t* desc;
     int64_t* segb;
-    uint32_t* sk;               // scratch pool: keys
-    int64_t* sv;                // scratch pool: values
+    PoolRow* pool;              // scratch pool
     unsigned long long* cnt;
     unsigned long long* sum;
     unsigned long long* mn;
@@ -554,8 +564,7 @@ __global__ void __launch_bounds__(kBThreads) k_batch_pass1(BArgs p, int32_t wave
                     if (!pass) return;
                     if (sbase >= 0) {
                         const uint32_t at = atomicAdd(&cur[key >> cbits], 1u);
-                        p.sk[sbase + at] = key;
-                        p.sv[sbase + at] = val;
+                        p.pool[sbase + at] = pool_row(key, val);
                     } else {
                         const uint64_t e = enc_i64(val);
                         add_global(p, Q.out + key, 1u, val, e, e);
@@ -579,8 +588,7 @@ __global__ void __launch_bounds__(kBThreads) k_batch_pass1(BArgs p, int32_t wave
                     const int64_t val = vv[j];
                     if (sbase >= 0) {
                         const uint32_t at = atomicAdd(&cur[key >> cbits], 1u);
-                        p.sk[sbase + at] = key;
-                        p.sv[sbase + at] = val;
+                        p.pool[sbase + at] = pool_row(key, val);
                     } else {
                         const uint64_t e = enc_i64(val);
                         add_global(p, Q.out + key, 1u, val, e, e);
@@ -648,8 +656,9 @@ __global__ void __launch_bounds__(kBThreads) k_batch_pass2(BArgs p, int32_t wave
 #pragma unroll
                 for (int u = 0; u < kU; u++) {
                     const int32_t i = min(i0 + u * 64 + lane, hi - 1);
-                    kk[u] = p.sk[base + i];
-                    vv[u] = p.sv[base + i];
+                    const PoolRow r = p.pool[base + i];
+                    kk[u] = r.w[0];
+                    vv[u] = (int64_t)((uint64_t)r.w[1] | ((uint64_t)r.w[2] << 32));
                 }
 #pragma unroll
                 for (int u = 0; u < kU; u++) {
@@ -747,9 +756,8 @@ struct qk_batch_s {
     int64_t desc_cap = 0;
     int64_t* segb = nullptr;
     int64_t segb_cap = 0;
-    uint32_t* sk = nullptr;
-    int64_t* sv = nullptr;
-    int64_t sk_cap = 0;
+    PoolRow* pool = nullptr;
+    int64_t pool_cap = 0;
     unsigned long long *cnt = nullptr, *sum = nullptr, *mn = nullptr, *mx = nullptr;  // owned results
     int64_t out_cap = 0;
     unsigned long long* res[4] = {};  // result arrays of the last run: owned or the caller's
@@ -833,17 +841,16 @@ void free_buffers(qk_batch_s* b) {
     b->owide = nullptr;
     b->bounds = nullptr;
     b->order_tiles = b->bound_blocks = 0;
-    void* ptrs[] = {b->units, b->desc, b->segb, b->sk, b->sv, b->cnt, b->sum, b->mn, b->mx};
+    void* ptrs[] = {b->units, b->desc, b->segb, b->pool, b->cnt, b->sum, b->mn, b->mx};
     for (void* p : ptrs)
         if (p) pool_free(p);
     b->units = nullptr;
     b->desc = nullptr;
     b->segb = nullptr;
-    b->sk = nullptr;
-    b->sv = nullptr;
+    b->pool = nullptr;
     b->cnt = b->sum = b->mn = b->mx = nullptr;
     for (auto& r : b->res) r = nullptr;
-    b->unit_cap = b->desc_cap = b->segb_cap = b->sk_cap = b->out_cap = 0;
+    b->unit_cap = b->desc_cap = b->segb_cap = b->pool_cap = b->out_cap = 0;
     if (b->host_units) (void)hipHostFree(b->host_units);
     b->host_units = nullptr;
     b->host_unit_cap = 0;
@@ -871,8 +878,7 @@ BArgs args_of(const qk_batch_s* b, bool ordered) {
     p.comp = b->comp;
     p.desc = b->desc;
     p.segb = b->segb;
-    p.sk = b->sk;
-    p.sv = b->sv;
+    p.pool = b->pool;
     p.cnt = b->res[0];
     p.sum = b->res[1];
     p.mn = b->res[2];
@@ -1187,19 +1193,16 @@ int run_batch(qk_batch_s* b, int32_t nq, const qk_batch_query* q, hipStream_t s,
     int64_t need_all = 0;
     for (int64_t e : b->est_host) need_all += e + e / 4 + 4096;
     const int64_t want = std::min(b->scratch_rows, need_all);
-    if (nlarge && (!b->sk || !b->sv || b->sk_cap < want)) {
+    if (nlarge && (!b->pool || b->pool_cap < want)) {
         free_graph(b);
-        const int64_t cap = std::min(b->scratch_rows, std::max(want, b->sk_cap + b->sk_cap / 2));
-        if (b->sk) pool_free(b->sk);
-        if (b->sv) pool_free(b->sv);
-        b->sk = nullptr;
-        b->sv = nullptr;
-        b->sk_cap = 0;
-        QK_TRY(pool_alloc((void**)&b->sk, (size_t)cap * 4));
-        QK_TRY(pool_alloc((void**)&b->sv, (size_t)cap * 8));
-        b->sk_cap = cap;
+        const int64_t cap = std::min(b->scratch_rows, std::max(want, b->pool_cap + b->pool_cap / 2));
+        if (b->pool) pool_free(b->pool);
+        b->pool = nullptr;
+        b->pool_cap = 0;
+        QK_TRY(pool_alloc((void**)&b->pool, (size_t)cap * sizeof(PoolRow)));
+        b->pool_cap = cap;
     }
-    const int64_t pool = b->sk_cap;
+    const int64_t pool = b->pool_cap;
     // chunks of the large queries
     const int64_t target = std::max<int64_t>((int64_t)1 << 18, pool / ((int64_t)device_info().cus * 4));
     int64_t desc = 0, segb = 0, chunk_units = 0;
@@ -1356,11 +1359,9 @@ int qk_batch_set_tuning(qk_batch b, const qk_batch_tuning* t) {
     b->tune = *t;
     const int64_t rows = t->scratch_rows > 0 ? t->scratch_rows : kDefaultScratchRows;
     if (rows != b->scratch_rows) {
-        if (b->sk) pool_free(b->sk);
-        if (b->sv) pool_free(b->sv);
-        b->sk = nullptr;
-        b->sv = nullptr;
-        b->sk_cap = 0;
+        if (b->pool) pool_free(b->pool);
+        b->pool = nullptr;
+        b->pool_cap = 0;
         b->scratch_rows = rows;
         free_graph(b);
     }
