@@ -17,8 +17,7 @@ namespace {
 
 constexpr int kBlock = 256;
 
-int grid_for(int64_t items, int per_block) {
-    const DeviceInfo& d = device_info();
+int grid_for(int64_t items, int per_block, const DeviceInfo& d = device_info()) {
     int64_t g = (items + per_block - 1) / per_block;
     int64_t cap = (int64_t)(d.cus > 0 ? d.cus : 64) * 16;
     if (g > cap) g = cap;
@@ -172,8 +171,9 @@ int launch_typed(bool bits, int32_t op, int32_t lkind, const void* lhs, int32_t 
                                                     (uint64_t*)out, n);
     } else {
         // 8 rows per lane; 4 while those would leave lanes of the chip without work
-        const bool wide = n >= (int64_t)device_info().cus * 2048 * 8;
-        const int grid = grid_for(wide ? n / 8 : (n + 3) / 4, kBlock);
+        const DeviceInfo& d = device_info();
+        const bool wide = n >= (int64_t)d.cus * 2048 * 8;
+        const int grid = grid_for(wide ? n / 8 : (n + 3) / 4, kBlock, d);
 #define QK_FILTER(AC, BC)                                                                                       \
     do {                                                                                                        \
         if (wide) k_filter_i8<L, R, AC, BC, 8><<<grid, kBlock, 0, s>>>(op, a, ac, b, bc, nm, (int8_t*)out, n);  \
