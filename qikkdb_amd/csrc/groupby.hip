@@ -869,8 +869,8 @@ LdsShape choose_lds(const qk_groupby_s* h) {
         while (L.rbits < kMaxCopyBits && lds_table_bytes(L.H, L.rbits + 1, h->fields) <= budget) L.rbits++;
         L.all = true;
         L.keys = (int64_t)h->logical_cap;
-        // two rows per entry: a workgroup's table then costs no more traffic than its rows
-        L.min_rows = 2 * (int64_t)L.H;
+        // four rows per entry: a workgroup's table then costs less traffic than its rows
+        L.min_rows = 4 * (int64_t)L.H;
     }
     return L;
 }

@@ -10,8 +10,10 @@
 // string owns one slot for the table's lifetime, and the slot's index is the string's int64 key
 // in an inner qk_groupby, which keeps every aggregate, NULL rule and path of the numeric table.
 // Per block:
-//   1. k_str_probe hashes each row's bytes (FNV-1a, 64 bits: the low bits pick the home slot,
-//      the high 32 bits are a tag kept in the slot word) and probes linearly.  A slot word is
+//   1. k_str_probe hashes each row's bytes by 8-byte words (the low bits pick the home slot, the
+//      high 32 bits are a tag kept in the slot word) and probes linearly, reading the slots through
+//      the caches (3M rows of 17 bytes, 700 strings: 385 us byte by byte and past the caches, 115 us
+//      so).  A slot word is
 //      0 (empty), tag | 1 (a string of an earlier block, its bytes in the table's arena), or
 //      tag | 2^31 | r (row r of this block, claimed by CAS in this kernel).  Equal tags are
 //      confirmed byte by byte against the arena or against the block's own input, which this
@@ -29,6 +31,7 @@
 namespace {
 
 constexpr uint32_t kRowBit = 0x80000000u;
+constexpr int32_t kLeadRows = 16384;
 
 struct StrDict {
     unsigned long long* slots;  // [D]
@@ -41,20 +44,57 @@ struct StrDict {
     unsigned long long* arena_used;
 };
 
-// FNV-1a over the bytes (Fowler, Noll and Vo's 64-bit offset basis and prime).
-__device__ __forceinline__ uint64_t str_hash(const char* p, int32_t len) {
-    uint64_t h = 0xcbf29ce484222325ull;
-    for (int32_t i = 0; i < len; i++) {
-        h ^= (uint8_t)p[i];
-        h *= 0x100000001b3ull;
-    }
-    return h;
+// ---- strings by 8-byte words ---------------------------------------------------------------
+//
+// A string is read as its full 8-byte words and a tail of the 0..7 bytes left, zero-extended.  The tail
+// comes from the 8 bytes that END with the string (they may begin in the string before it), so no read
+// passes the end of the buffer; strings ending within the buffer's first 8 bytes are read byte by byte.
+// The hardware takes 8-byte loads at any address.
+
+__device__ __forceinline__ uint64_t str_word(const char* p) {
+    uint64_t w;
+    __builtin_memcpy(&w, qk::to_g(p), 8);
+    return w;
 }
 
-__device__ __forceinline__ bool str_eq(const char* a, const char* b, int32_t len) {
-    for (int32_t i = 0; i < len; i++)
-        if (a[i] != b[i]) return false;
-    return true;
+// The last `rem` (1..7) bytes of a string that ends at buf + end.
+__device__ __forceinline__ uint64_t str_tail(const char* buf, int64_t end, int rem) {
+    if (end >= 8) return str_word(buf + end - 8) >> (64 - 8 * rem);
+    uint64_t w = 0;
+    for (int i = 0; i < rem; i++) w |= (uint64_t)(uint8_t)buf[end - rem + i] << (8 * i);
+    return w;
+}
+
+// Multiplies by 2^64 / golden ratio and folds the high half down, so that every word's bits reach both
+// the slot (low) and the tag (high) bits.
+__device__ __forceinline__ uint64_t str_mix(uint64_t h, uint64_t w) {
+    h = (h ^ w) * 0x9e3779b97f4a7c15ull;
+    return h ^ (h >> 29);
+}
+
+__device__ __forceinline__ uint64_t str_hash(const char* buf, int64_t start, int32_t len) {
+    const int32_t words = len >> 3, rem = len & 7;
+    uint64_t h = str_mix(0x5bd1e9955bd1e995ull, (uint64_t)len);
+    constexpr int kAhead = 4;  // words loaded together
+    for (int32_t i0 = 0; i0 < words; i0 += kAhead) {
+        uint64_t w[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; i++) w[i] = str_word(buf + start + 8 * min(i0 + i, words - 1));
+#pragma unroll
+        for (int i = 0; i < kAhead; i++)
+            if (i0 + i < words) h = str_mix(h, w[i]);
+    }
+    if (rem) h = str_mix(h, str_tail(buf, start + len, rem));
+    return str_mix(h, h >> 32);
+}
+
+// Whether two strings of the same length are equal.
+__device__ __forceinline__ bool str_eq(const char* a, int64_t as, const char* b, int64_t bs, int32_t len) {
+    const int32_t words = len >> 3, rem = len & 7;
+    uint64_t diff = 0;
+    for (int32_t i = 0; i < words && !diff; i++) diff = str_word(a + as + 8 * i) ^ str_word(b + bs + 8 * i);
+    if (rem && !diff) diff = str_tail(a, as + len, rem) ^ str_tail(b, bs + len, rem);
+    return diff == 0;
 }
 
 __device__ __forceinline__ int64_t str_start(const int64_t* idx, int64_t i) { return i ? idx[i - 1] : 0; }
@@ -67,22 +107,23 @@ __global__ void k_str_arm(StrDict d) {
 // or (with counters[1] set) a row whose string found no free slot.
 __global__ void __launch_bounds__(256) k_str_probe(StrDict d, const char* __restrict__ chars,
                                                    const int64_t* __restrict__ idx,
-                                                   const uint64_t* __restrict__ knull, int32_t n,
+                                                   const uint64_t* __restrict__ knull, int32_t row0, int32_t n,
                                                    qk::PredSet preds, int64_t* __restrict__ out_slot) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    for (int64_t i = row0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         int64_t res = -1;
         bool pass = !(knull && qk::null_bit(knull, i));
         for (int p = 0; p < preds.n && pass; p++) pass = qk::eval_pred(preds.p[p], i);
         if (pass) {
             const int64_t start = str_start(idx, i);
             const int32_t len = (int32_t)(idx[i] - start);
-            const char* s = chars + start;
-            const uint64_t h = str_hash(s, len);
+            const uint64_t h = str_hash(chars, start, len);
             const unsigned long long tag = h & 0xffffffff00000000ull;
             uint64_t pos = h & d.mask;
             for (uint64_t pr = 0; pr <= d.mask; pr++) {
-                unsigned long long w = *(volatile unsigned long long*)(d.slots + pos);
+                // read through the caches: a word only ever changes from empty, and what seems empty is
+                // settled by the CAS
+                unsigned long long w = qk::to_g(d.slots)[pos];
                 if (w == 0ull) {
                     w = atomicCAS(d.slots + pos, 0ull, tag | kRowBit | (unsigned long long)i);
                     if (w == 0ull) {
@@ -93,18 +134,11 @@ __global__ void __launch_bounds__(256) k_str_probe(StrDict d, const char* __rest
                 }
                 if ((w & 0xffffffff00000000ull) == tag) {
                     const uint32_t low = (uint32_t)w;
-                    const char* o;
-                    int32_t olen;
-                    if (low & kRowBit) {
-                        const int64_t r = low & ~kRowBit;
-                        const int64_t os = str_start(idx, r);
-                        o = chars + os;
-                        olen = (int32_t)(idx[r] - os);
-                    } else {
-                        o = d.arena + d.off[pos];
-                        olen = d.len[pos];
-                    }
-                    if (olen == len && str_eq(o, s, len)) {
+                    const bool row = (low & kRowBit) != 0;
+                    const int64_t r = low & ~kRowBit;
+                    const int64_t os = row ? str_start(idx, r) : d.off[pos];
+                    const int32_t olen = row ? (int32_t)(idx[r] - os) : d.len[pos];
+                    if (olen == len && str_eq(row ? chars : d.arena, os, chars, start, len)) {
                         res = (int64_t)pos;
                         break;
                     }
@@ -327,7 +361,12 @@ int gbs_block(qk_gbs_s* h, const char* chars, const int64_t* indices, const uint
     QK_TRY(gbs_reserve(h, n, total, s));
     StrDict d = view(h);
     k_str_arm<<<1, 64, 0, s>>>(d);
-    k_str_probe<<<grid_for(n), 256, 0, s>>>(d, chars, indices, key_nulls, n, ps, h->slot_col);
+    // the block's first rows on their own: they bring its frequent strings into the dictionary, and the
+    // next launch then finds them through the caches; a string that is inserted while others look for it
+    // looks absent in every cache that has read its slot before, and each look costs a CAS
+    const int32_t lead = std::min(n, kLeadRows);
+    k_str_probe<<<grid_for(lead), 256, 0, s>>>(d, chars, indices, key_nulls, 0, lead, ps, h->slot_col);
+    if (lead < n) k_str_probe<<<grid_for(n - lead), 256, 0, s>>>(d, chars, indices, key_nulls, lead, n, ps, h->slot_col);
     k_str_commit<<<grid_for(n), 256, 0, s>>>(d, chars, indices);
     QK_HIP(hipGetLastError());
     h->arena_bound += total;
