@@ -328,8 +328,12 @@ ValueRange range_of(const Fold& f) {
     return vr;
 }
 
-bool foldable_op(int32_t op) {
-    return op == QK_GREATER || op == QK_GREATER_EQUAL || op == QK_LESS || op == QK_LESS_EQUAL || op == QK_EQUAL;
+// Whether a comparison with a constant folds into an interval.  Nothing compares true with a NaN constant,
+// which no interval says.
+bool foldable(const qk_predicate& p) {
+    const bool op = p.op == QK_GREATER || p.op == QK_GREATER_EQUAL || p.op == QK_LESS || p.op == QK_LESS_EQUAL ||
+                    p.op == QK_EQUAL;
+    return p.rhs_kind == QK_CONST && op && !(is_real_type(p.rhs_type) && p.rhs_real != p.rhs_real);
 }
 
 }  // namespace
@@ -339,7 +343,7 @@ bool fold_value_range(PredSet* ps, uint32_t vpred, int32_t vtype) {
     Fold f;
     for (int i = 0; i < ps->n; i++) {
         const qk_predicate& p = ps->p[i];
-        if (!((vpred >> i) & 1u) || p.rhs_kind != QK_CONST || !foldable_op(p.op)) return false;
+        if (!((vpred >> i) & 1u) || !foldable(p)) return false;
         switch (vtype) {
         case QK_INT: fold_typed<int32_t>(p, f); break;
         case QK_LONG: fold_typed<int64_t>(p, f); break;
@@ -359,8 +363,7 @@ bool fold_column_range(PredSet* ps, uint32_t vpred) {
     Fold f;
     for (int i = 0; i < ps->n; i++) {
         const qk_predicate& p = ps->p[i];
-        if (p.column != p0.column || p.type != p0.type || p.null_mask != p0.null_mask || p.rhs_kind != QK_CONST ||
-            !foldable_op(p.op))
+        if (p.column != p0.column || p.type != p0.type || p.null_mask != p0.null_mask || !foldable(p))
             return false;
         if (p0.type == QK_INT) fold_typed<int32_t>(p, f); else fold_typed<int64_t>(p, f);
     }
@@ -377,8 +380,7 @@ void fold_columns(const PredSet& ps, RangeSet* rs, PredSet* rest) {
     rest->n = 0;
     for (int i = 0; i < ps.n; i++) {
         const qk_predicate& p = ps.p[i];
-        // nothing compares true with a NaN constant, which no interval says
-        if (p.rhs_kind != QK_CONST || !foldable_op(p.op) || (is_real_type(p.rhs_type) && p.rhs_real != p.rhs_real)) {
+        if (!foldable(p)) {
             rest->p[rest->n++] = p;
             continue;
         }

@@ -25,6 +25,7 @@
 #include "groupby.hpp"
 #include "ldstable.hpp"
 #include "lookback.hpp"
+#include "rowstream.hpp"
 #include "twophase.hpp"
 
 namespace qk {
@@ -518,6 +519,64 @@ __global__ void __launch_bounds__(256) k_gb_merge(GView dst, GView src, uint32_t
     if (threadIdx.x == 0) g_count_new(dst, s_new);
 }
 
+// Slot ids of a block's rows for the two phases over a multi-word table: a row that passes the WHERE
+// (int8 mask, folded columns and the predicates left over) gets the slot of its key, claimed when absent,
+// any other -1.  Rows [row0, n).  Bound by the 16-byte reads of the key table, through the caches.
+template <int KW>
+__global__ void __launch_bounds__(512) k_gb_ids(GView g, KeySpec ks, KeyCols kc, const int8_t* __restrict__ mask,
+                                                RangeSet rs, PredSet rest, int64_t row0, int64_t n,
+                                                int32_t* __restrict__ ids) {
+    __shared__ unsigned int s_new;
+    if (threadIdx.x == 0) s_new = 0;
+    __syncthreads();
+    const int64_t tile_rows = (int64_t)blockDim.x * kSteps;
+    for (int64_t base = row0 + blockIdx.x * tile_rows; base < n; base += gridDim.x * tile_rows) {
+        int64_t r[kSteps];
+        bool ok[kSteps], kn[kSteps];
+        uint64_t key[kSteps][KW];
+#pragma unroll
+        for (int k = 0; k < kSteps; k++) {
+            const int64_t row = base + k * (int64_t)blockDim.x + threadIdx.x;
+            ok[k] = row < n;
+            r[k] = min(row, n - 1);
+        }
+        load_keys<KW, kSteps>(ks, kc, r, key, kn);
+        if (mask) {
+#pragma unroll
+            for (int k = 0; k < kSteps; k++) ok[k] = ok[k] & (mask[r[k]] != 0);
+        }
+        for (int i = 0; i < rs.n; i++) rows_in_range<kSteps>(rs.c[i], r, ok);
+        for (int p = 0; p < rest.n; p++)
+#pragma unroll
+            for (int k = 0; k < kSteps; k++)
+                if (ok[k]) ok[k] = eval_pred(rest.p[p], r[k]);
+        u64x2 tail[kSteps];
+        uint64_t home[kSteps];
+#pragma unroll
+        for (int k = 0; k < kSteps; k++) {
+            home[k] = home_of(g, key_hash<KW>(key[k]));
+            tail[k] = g_key_tail<KW>(g, home[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < kSteps; k++) {
+            int64_t gs = -1;
+            if (ok[k]) {
+                gs = g_find_cached<KW>(g, key[k], home[k], tail[k]);
+                if (gs < 0) {
+                    bool is_new = false;
+                    gs = g_slotN<KW>(g, key[k], key_hash<KW>(key[k]), &is_new);
+                    if (is_new) atomicAdd(&s_new, 1u);
+                    if (gs < 0) g_set_lost(g);
+                }
+            }
+            const int64_t row = base + k * (int64_t)blockDim.x + threadIdx.x;
+            if (row < n) ids[row] = (int32_t)gs;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) g_count_new(g, s_new);
+}
+
 // Rows of a block still to aggregate after the table dropped partials (a growing table): rows
 // that pass the block's WHERE (MODE 0 none, 1 int8 mask, 2 predicate list) and whose key the
 // table does not hold.  out[r] = 1 for those rows, 0 otherwise.  `out` may be `mask` itself
@@ -622,6 +681,7 @@ struct qk_groupby_s {
     uint64_t cap = 0;
     int32_t parts = 1;      // sub-tables of the hashed slots
     int32_t rec_parts = 1;  // partitions of the two-phase path's cold rows (divides parts)
+    int32_t id_parts = 0;   // multi-word keys: slot ranges of the two-phase path (0: not taken)
     bool real_sum = false;
     // storage (structure of arrays)
     uint64_t* keys = nullptr;
@@ -708,6 +768,38 @@ void layout_table(qk_groupby_s* h, uint64_t logical) {
     }
     h->parts = parts;
     h->rec_parts = std::min<int32_t>(parts, kMaxRecParts);
+    h->id_parts = 0;
+    if (h->ks.kw > 1) {
+        // two phases over the slots: up to 256 ranges of at least 64 slots, more where a range's
+        // states would not fit the LDS
+        const size_t budget = std::min<size_t>(device_info().lds_per_block, 160 * 1024) - 512;
+        int64_t f = 1;
+        while (f < 256 && cap / (uint64_t)(f * 2) >= 64) f *= 2;
+        while (f < ((int64_t)kMaxRecParts << kMaxSplitBits) && p2d_lds_bytes((int64_t)(cap / (uint64_t)f), h->fields) > budget)
+            f *= 2;
+        if (p2d_lds_bytes((int64_t)(cap / (uint64_t)f), h->fields) <= budget) {
+            h->id_parts = (int32_t)f;
+            h->rec_parts = std::min<int32_t>((int32_t)f, kMaxRecParts);
+        }
+    }
+}
+
+int log2_of(uint64_t x) {
+    int b = 0;
+    while (((uint64_t)1 << b) < x) b++;
+    return b;
+}
+
+// The table as the two phases see it: a multi-word table's slots cut into id_parts ranges.
+GView phase_view(const qk_groupby_s* h) {
+    GView g = view_of(h);
+    if (h->ks.kw > 1 && h->id_parts > 0) {
+        const int pbits = log2_of((uint64_t)h->id_parts);
+        g.part_shift = 64 - pbits;
+        g.sub_bits = log2_of(h->cap) - pbits;
+        g.sub_mask = ((uint64_t)1 << g.sub_bits) - 1;
+    }
+    return g;
 }
 
 // Slot arrays for h->cap (+ 2 side slots); on failure every array is released.
@@ -764,7 +856,7 @@ int init_table(qk_groupby_s* h, hipStream_t s) {
 // Merge rows whose phase 2 was deferred; everything that reads the table calls this first.
 int flush_pending(qk_groupby_s* h, hipStream_t s) {
     if (h->tp.pending_rows == 0) return QK_SUCCESS;
-    return twophase_flush(h->tp, view_of(h), h->fields, s);
+    return twophase_flush(h->tp, phase_view(h), h->fields, s);
 }
 
 int read_counters(qk_groupby_s* h, hipStream_t s, TableCounters* out) {
@@ -808,7 +900,7 @@ int grow_table(qk_groupby_s* h, uint64_t need, hipStream_t s) {
     keep.mx = h->mx;
     const uint64_t old_logical = h->logical_cap;
     const uint64_t old_cap = h->cap;
-    const int32_t old_parts = h->parts, old_rec = h->rec_parts, old_max = h->reported_max;
+    const int32_t old_parts = h->parts, old_rec = h->rec_parts, old_max = h->reported_max, old_ids = h->id_parts;
     uint64_t logical = old_logical * 2;
     while (logical < need && logical < kMaxLogical) logical *= 2;
     layout_table(h, std::min<uint64_t>(logical, kMaxLogical));
@@ -824,6 +916,7 @@ int grow_table(qk_groupby_s* h, uint64_t need, hipStream_t s) {
         h->cap = old_cap;
         h->parts = old_parts;
         h->rec_parts = old_rec;
+        h->id_parts = old_ids;
         h->reported_max = old_max;
         return st;
     }
@@ -915,6 +1008,27 @@ void partials_for(qk_groupby_s* h, LdsShape* L, hipStream_t s) {
     L->part.mx = next(h->fields & F_MAX);
 }
 
+// The slot ids of a block.  Its first rows go ahead on their own: they bring the frequent keys into the
+// table, and the next launch then finds them through the caches (a key that is inserted while others look
+// for it looks absent in every cache that has read its slot before).
+int launch_ids(const qk_groupby_s* h, const GView& g, const KeyCols& kc, const int8_t* mask, const PredSet& ps,
+               int64_t n, int32_t* ids, hipStream_t s) {
+    constexpr int64_t kLead = 65536;
+    constexpr int kIdBlock = 512;
+    RangeSet rs{};
+    PredSet rest{};
+    fold_columns(ps, &rs, &rest);
+    for (int64_t r0 = 0; r0 < n; r0 = r0 == 0 ? std::min(n, kLead) : n) {
+        const int64_t r1 = r0 == 0 ? std::min(n, kLead) : n;
+        const unsigned grid = (unsigned)std::min<int64_t>((r1 - r0 + kIdBlock * kSteps - 1) / (kIdBlock * kSteps),
+                                                          (int64_t)device_info().cus * 8);
+        if (h->ks.kw == 2) k_gb_ids<2><<<grid, kIdBlock, 0, s>>>(g, h->ks, kc, mask, rs, rest, r0, r1, ids);
+        else k_gb_ids<4><<<grid, kIdBlock, 0, s>>>(g, h->ks, kc, mask, rs, rest, r0, r1, ids);
+        QK_HIP(hipGetLastError());
+    }
+    return QK_SUCCESS;
+}
+
 std::pair<hipEvent_t, hipEvent_t>* next_events(qk_groupby h) {
     if (h->events_used == h->events.size()) {
         hipEvent_t a, b;
@@ -959,7 +1073,8 @@ int process_once(qk_groupby h, int mode, const void* const* keys, const uint64_t
     const int vtype = values ? h->value_type : 0;
     // a table whose every key fits a workgroup's LDS takes the one-pass kernel at any size
     LdsShape L = choose_lds(h);
-    const bool two = twophase_supported(h->ks.kw, h->value_type) &&
+    const bool ids = h->ks.kw > 1;
+    const bool two = (ids ? h->id_parts > 0 : twophase_supported(h->ks.kw, h->value_type)) &&
                      (h->twophase_mode == 1 ||
                       (h->twophase_mode < 0 && n >= h->twophase_min_rows && !L.all));
     int st;
@@ -969,18 +1084,53 @@ int process_once(qk_groupby h, int mode, const void* const* keys, const uint64_t
         // growing table grows at the block that filled it.
         const bool defer = (h->flags & (QK_GB_ASYNC | QK_GB_AUTO_GROW)) == QK_GB_ASYNC && h->tp.defer_rows != 0;
         TwoPhaseBufs& tp = h->tp;
+        const GView gp = phase_view(h);
+        const int32_t id_shift = ids ? 64 - log2_of(h->cap) : 0;
+        if (tp.id_shift != id_shift) {  // the table's first such block, or it has grown (nothing is pending)
+            if (tp.r_rec) {
+                QK_HIP(hipDeviceSynchronize());
+                twophase_free(tp);
+            }
+            tp.id_shift = id_shift;
+        }
         if (tp.pending_rows > 0 &&
             (twophase_needs_realloc(tp, h->rec_parts, h->value_type, values != nullptr, n, defer) ||
              tp.pending_rows + n > tp.rows_alloc || tp.pend_vtype != vtype))
-            QK_TRY(twophase_flush(tp, g, h->fields, s));
+            QK_TRY(twophase_flush(tp, gp, h->fields, s));
         QK_TRY(twophase_prepare(tp, h->rec_parts, h->fields, h->value_type, values != nullptr, n, defer, s));
+        // the rows as the phases read them: the block's columns, or its slot ids (the WHERE is done then)
+        KeySpec pks = h->ks;
+        KeyCols pkc = kc;
+        PredSet pps = ps;
+        int pmode = mode;
+        const int8_t* pmask = mask;
+        if (ids) {
+            QK_TRY(launch_ids(h, g, kc, mode == 1 ? mask : nullptr, ps, n, tp.ids, s));
+            pks = KeySpec{};
+            pks.nkeys = pks.kw = pks.single = 1;
+            pks.type[0] = QK_INT;
+            pkc = KeyCols{};
+            pkc.col[0] = tp.ids;
+            pps = PredSet{};
+            pmode = 0;
+            pmask = nullptr;
+        }
         if (!tp.heavy_ready)
-            QK_TRY(twophase_sample(tp, g, h->ks, kc, vtype, values, value_nulls, mask, ps, vpred, n, mode, s));
+            QK_TRY(twophase_sample(tp, gp, pks, pkc, vtype, values, value_nulls, pmask, pps, ids ? 0 : vpred, n, pmode, s));
         h->last_H = tp.H1;
         h->last_path = 1;
-        st = twophase_phase1(tp, g, h->ks, kc, vtype, values, value_nulls, mask, ps, vpred, n,
-                             h->fields, mode, s, ev ? ev->first : nullptr, ev ? ev->second : nullptr);
-        if (st == QK_SUCCESS && !defer) st = twophase_flush(tp, g, h->fields, s);
+        // slot ids are always streamed, in pieces of what the streaming reader can address
+        const int64_t piece = ids ? kStreamMaxRows : (int64_t)n;
+        st = QK_SUCCESS;
+        for (int64_t r0 = 0; r0 < n && st == QK_SUCCESS; r0 += piece) {
+            const void* v = values ? (const char*)values + r0 * type_size(h->value_type) : nullptr;
+            if (ids) pkc.col[0] = tp.ids + r0;
+            st = twophase_phase1(tp, gp, pks, pkc, vtype, v, value_nulls ? value_nulls + r0 / 64 : nullptr, pmask, pps,
+                                 ids ? 0 : vpred, std::min<int64_t>(piece, n - r0), h->fields, pmode, s,
+                                 ev && r0 == 0 ? ev->first : nullptr,
+                                 ev && r0 + piece >= n ? ev->second : nullptr);
+        }
+        if (st == QK_SUCCESS && !defer) st = twophase_flush(tp, gp, h->fields, s);
     } else {
         if (L.all) partials_for(h, &L, s);
         h->last_H = L.H;

@@ -137,6 +137,31 @@ struct RangeSet {
     RangeCol c[kMaxPreds];
 };
 
+// ok[k] of N rows (all inside the block) against one folded column: the column's loads are issued
+// together, the type switch is outside the rows.
+template <typename T, int N>
+__device__ __forceinline__ void rows_in_range_t(const RangeCol& c, const int64_t (&r)[N], bool (&ok)[N]) {
+    T v[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) v[k] = __builtin_nontemporal_load((const T*)c.col + r[k]);
+#pragma unroll
+    for (int k = 0; k < N; k++) ok[k] = ok[k] & in_range<T>(c.vr, v[k]);
+}
+template <int N>
+__device__ __forceinline__ void rows_in_range(const RangeCol& c, const int64_t (&r)[N], bool (&ok)[N]) {
+    if (c.nm) {
+#pragma unroll
+        for (int k = 0; k < N; k++) ok[k] = ok[k] & !null_bit(c.nm, r[k]);
+    }
+    switch (c.type) {
+    case QK_INT8: rows_in_range_t<int8_t, N>(c, r, ok); break;
+    case QK_INT: rows_in_range_t<int32_t, N>(c, r, ok); break;
+    case QK_LONG: rows_in_range_t<int64_t, N>(c, r, ok); break;
+    case QK_FLOAT: rows_in_range_t<float, N>(c, r, ok); break;
+    default: rows_in_range_t<double, N>(c, r, ok); break;
+    }
+}
+
 // The folded range column at row r, widened to int64.
 __device__ __forceinline__ int64_t range_col(const PredSet& ps, int64_t r) {
     return ps.rwide ? __builtin_nontemporal_load((const int64_t*)ps.rcol + r)

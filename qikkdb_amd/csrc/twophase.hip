@@ -50,6 +50,11 @@ __device__ __forceinline__ void get_rec(const uint32_t* base, int64_t at, uint64
     if constexpr (VTraits<VT>::has) __builtin_memcpy(&v, &r.w[2], sizeof(VT)); else v = 0;
 }
 
+// What places a key: its hash, or, for slot ids, the id at the top of the word.
+__device__ __forceinline__ uint64_t place_of(uint64_t k, int32_t id_shift) {
+    return id_shift ? k << id_shift : hash64(k);
+}
+
 // Exclusive prefix sum over the threads of a workgroup (blockDim a multiple of 64, <= 1024);
 // *total receives the sum.  `wsum` is LDS for 16 values.  Every thread must call it.
 __device__ __forceinline__ int32_t block_excl_scan(int32_t v, int32_t* wsum, int32_t* total) {
@@ -109,7 +114,7 @@ __global__ void __launch_bounds__(kSampleBlock) k_tp_sample(KeySpec ks, KeyCols 
                                                    const int8_t* __restrict__ mask, PredSet preds,
                                                    uint32_t vpred, int64_t n, int64_t stride,
                                                    int64_t nsamples, uint64_t* skeys,
-                                                   uint32_t* scnt, uint64_t smask) {
+                                                   uint32_t* scnt, uint64_t smask, int32_t id_shift) {
     __shared__ uint64_t lk[kSampleLds];
     __shared__ uint32_t lc[kSampleLds];
     for (int s = threadIdx.x; s < kSampleLds; s += blockDim.x) {
@@ -151,6 +156,7 @@ __global__ void __launch_bounds__(kSampleBlock) k_tp_sample(KeySpec ks, KeyCols 
         for (int u = 0; u < kBatch; u++) {
         if (!ok[u] || !row_passes<VT, MODE>(preds, vpred, mask, rr[u], v[u], vn[u], cv[u], cn[u])) continue;
         if (kn[u] || k[u][0] == kEmpty) continue;  // those keys have side slots anyway
+        if (id_shift && (int64_t)k[u][0] < 0) continue;
         const uint64_t key = k[u][0];
         uint32_t s = (uint32_t)(hash64(key) >> 53) & (kSampleLds - 1);
         bool done = false;
@@ -284,7 +290,7 @@ __device__ __forceinline__ uint32_t bucket_of(uint64_t k, uint32_t nb) {
 // Dynamic LDS: H keys of the table + kmax keys and counts of the ordered set.
 __global__ void __launch_bounds__(1024) k_tp_order(const uint64_t* __restrict__ cand,
                                                    const uint32_t* __restrict__ cand_cnt, int32_t kmax,
-                                                   int32_t P, int32_t part_shift, int32_t* meta,
+                                                   int32_t P, int32_t part_shift, int32_t id_shift, int32_t* meta,
                                                    uint64_t* __restrict__ heavy, uint32_t* __restrict__ heavy_cnt,
                                                    int32_t H, uint64_t* __restrict__ image,
                                                    int32_t* __restrict__ slot) {
@@ -301,7 +307,7 @@ __global__ void __launch_bounds__(1024) k_tp_order(const uint64_t* __restrict__ 
     for (int i = t; i < H; i += bd) lkey[i] = kEmpty;
     __syncthreads();
     for (int i = t; i < K; i += bd) {
-        const uint64_t h = hash64(cand[i]);
+        const uint64_t h = place_of(cand[i], id_shift);
         const int p = part_shift >= 64 ? 0 : (int)(h >> part_shift);
         atomicAdd(&cnt[p], 1);
     }
@@ -319,7 +325,7 @@ __global__ void __launch_bounds__(1024) k_tp_order(const uint64_t* __restrict__ 
     __syncthreads();
     for (int i = t; i < K; i += bd) {
         const uint64_t key = cand[i];
-        const uint64_t h = hash64(key);
+        const uint64_t h = place_of(key, id_shift);
         const int p = part_shift >= 64 ? 0 : (int)(h >> part_shift);
         const int32_t at = atomicAdd(&cur[p], 1);
         heavy[at] = key;
@@ -391,6 +397,7 @@ struct P1Args {
     uint32_t* r_count;
     const uint64_t* zero;  // a zero word (stands in for an absent null bitmap)
     int32_t part_shift;    // partition of a key hash: h >> part_shift (0 when >= 64)
+    int32_t id_shift;      // slot ids: place_of
     int32_t accumulate;    // regions and partials hold rows of earlier blocks
 };
 
@@ -557,13 +564,13 @@ __device__ __forceinline__ void p1_heavy_add(const P1Lds<VV>& L, int l, const VV
 // A row that cannot go to a region (NULL value, or its region is full): straight into the
 // global table with atomics.
 template <typename VT, typename VV>
-__device__ __forceinline__ void p1_atomic_row(const GView* gp, uint32_t* nnew, uint32_t fields, uint64_t kk,
-                                              uint64_t h, const VV& v, bool vn) {
+__device__ __forceinline__ void p1_atomic_row(const GView* gp, uint32_t* nnew, uint32_t fields, int32_t id_shift,
+                                              uint64_t kk, const VV& v, bool vn) {
     Part pr;
     if constexpr (VTraits<VT>::has) pr = row_part<VT>(v, vn); else pr = row_part<NoValue>(NoValue{}, vn);
     const GView& g = *gp;
     bool is_new = false;
-    const int64_t gs = g_slot1(g, kk, false, h, &is_new);
+    const int64_t gs = id_shift ? (int64_t)kk : g_slot1(g, kk, false, hash64(kk), &is_new);
     if (is_new) atomicAdd(nnew, 1u);
     if (gs >= 0) g_accum_atomic(g, gs, pr, fields); else g_set_lost(g);
 }
@@ -583,7 +590,7 @@ struct P1Ring {
         const uint64_t kk = L.qkey[at_q];
         VV v = 0;
         if constexpr (VTraits<VT>::has) v = L.qval[at_q];
-        const uint64_t h = hash64(kk);
+        const uint64_t h = place_of(kk, a.id_shift);
         // part_shift is 54..64; the split shift gives 0 for 64 without a select
         const uint32_t q = (uint32_t)((h >> 1) >> (a.part_shift - 1));
         uint32_t c = ~0u;
@@ -591,7 +598,7 @@ struct P1Ring {
         if (live && c < (uint32_t)a.cap) {
             put_rec<VT>(a.r_rec, ((int64_t)blockIdx.x * a.P + q) * (int64_t)a.cap + c, kk, v);
         } else if (live) {
-            p1_atomic_row<VT>(gp, L.nnew, fields, kk, h, v, false);
+            p1_atomic_row<VT>(gp, L.nnew, fields, a.id_shift, kk, v, false);
         }
         head = (head + n) & (kQueue - 1);
     }
@@ -736,7 +743,7 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase1(const GView* gp, KeySpec k
         for (int k = 0; k < kP1Steps; k++) {
             const bool pass = (o.pass >> k) & 1, vn = (o.vnull >> k) & 1;
             const bool cold = pass & (ls[k] < 0);
-            if (cold && vn) p1_atomic_row<VT>(gp, L.nnew, fields, o.key[k], hash64(o.key[k]), o.val[k], true);
+            if (cold && vn) p1_atomic_row<VT>(gp, L.nnew, fields, 0, o.key[k], o.val[k], true);
             ring.push(L, a, gp, fields, cold && !vn, o.key[k], o.val[k]);
         }
     };
@@ -776,21 +783,25 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase1s(const GView* gp, KeyCols 
         // equal to the empty marker then take their side slots by selection); with no heavy key
         // the table is not read
         int ls[kSRows];
+        bool pass[kSRows];
 #pragma unroll
         for (int j = 0; j < kSRows; j++) {
+            // a slot id of -1 is a row that the WHERE dropped
+            pass[j] = o.pass[j];
+            if constexpr (std::is_same<KT, int32_t>::value) pass[j] = pass[j] & !(a.id_shift && (int64_t)o.key[j] < 0);
             int l = K ? heavy_find(L.lkey, nb, o.key[j]) : -1;
             l = o.key[j] == kEmpty ? H + 1 : l;
             ls[j] = o.knull[j] ? H : l;
         }
 #pragma unroll
         for (int j = 0; j < kSRows; j++)
-            if (o.pass[j] && ls[j] >= 0) p1_heavy_add<VT>(L, ls[j], o.val[j], o.vnull[j]);
+            if (pass[j] && ls[j] >= 0) p1_heavy_add<VT>(L, ls[j], o.val[j], o.vnull[j]);
         // cold rows with a value go to the ring; a NULL value takes the atomic path
 #pragma unroll
         for (int j = 0; j < kSRows; j++) {
-            const bool cold = o.pass[j] & (ls[j] < 0);
+            const bool cold = pass[j] & (ls[j] < 0);
             if (cold && o.vnull[j])
-                p1_atomic_row<VT>(gp, L.nnew, fields, o.key[j], hash64(o.key[j]), o.val[j], true);
+                p1_atomic_row<VT>(gp, L.nnew, fields, a.id_shift, o.key[j], o.val[j], true);
             ring.push(L, a, gp, fields, cold && !o.vnull[j], o.key[j], o.val[j]);
         }
     });
@@ -812,6 +823,7 @@ struct P2Args {
     const uint32_t* r_rec;
     const uint32_t* r_count;
     int32_t split;  // log2(sub-tables per partition), owned phase 2 only
+    int32_t id_shift;
 };
 
 __host__ __device__ inline size_t p2_lds_bytes(int32_t H2, int32_t W, uint32_t fields) {
@@ -1105,7 +1117,10 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase2(GView g, uint32_t fields, 
 // and no row needs a global probe or atomic.  Counts are 32-bit deltas (one flush holds at
 // most 2^30 rows); the global states stay 64-bit.  The kernel has no static LDS, so the
 // sub-table may use all of it.
-template <typename VT, int FP>
+//
+// IDS: the keys are slot ids of a multi-word table; a row's place is known, and the sub-table's keys
+// are neither read nor written.
+template <typename VT, int FP, bool IDS>
 __global__ void __launch_bounds__(kBlock) k_tp_phase2_owned(GView g, uint32_t fields, P2Args a) {
     extern __shared__ __align__(16) uint64_t lds[];
     constexpr bool HAS_V = VTraits<VT>::has;
@@ -1131,7 +1146,10 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase2_owned(GView g, uint32_t fi
     const int64_t base = (int64_t)part << g.sub_bits;
     // 8-byte arrays first, then the 4-byte ones
     uint64_t* okey = lds;
-    unsigned long long* p = (unsigned long long*)(okey + S);
+    unsigned long long* p = (unsigned long long*)(IDS ? lds : okey + S);
+    // the slots' hash (or id) of a key, and its home slot in the sub-table
+    auto place = [&](uint64_t key) { return IDS ? key << a.id_shift : hash64(key); };
+    auto home_in = [&](uint64_t key, uint64_t h) { return (uint32_t)((IDS ? key : h) & g.sub_mask); };
     unsigned long long* osum = f_sum ? p : nullptr;
     p += f_sum ? S : 0;
     unsigned long long* omin = f_min ? p : nullptr;
@@ -1148,13 +1166,13 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase2_owned(GView g, uint32_t fi
 #pragma unroll
         for (int u = 0; u < kFill; u++) {
             const uint32_t s = s0 + u * bd;
-            k[u] = s < S ? g.keys[base + s] : 0ull;
+            k[u] = !IDS && s < S ? g.keys[base + s] : 0ull;
         }
 #pragma unroll
         for (int u = 0; u < kFill; u++) {
             const uint32_t s = s0 + u * bd;
             if (s >= S) continue;
-            okey[s] = k[u];
+            if (!IDS) okey[s] = k[u];
             ocnt[s] = 0;
             if (oall) oall[s] = 0;
             if (osum) osum[s] = 0;
@@ -1168,6 +1186,7 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase2_owned(GView g, uint32_t fi
     // slot of a key (claimed when absent), probing from h & sub_mask as g_slot1 does
     // (free: slot s was seen empty, so the claim starts with the CAS)
     auto claim_from = [&](uint64_t key, uint32_t s, bool free = false) -> int {
+        if (IDS) return (int)s;
         for (uint32_t it = 0; it < S; it++) {
             const uint64_t cur = free ? kEmpty : okey[s];
             free = false;
@@ -1212,7 +1231,7 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase2_owned(GView g, uint32_t fi
             const int w0 = nk <= bd ? tid / nk : 0;
             for (int ki = nk <= bd ? tid % nk : tid; ki < nk; ki += (nk <= bd ? nk : bd)) {
                 const uint64_t key = a.heavy[hk0 + ki];
-                const uint64_t kh = hash64(key);
+                const uint64_t kh = place(key);
                 if (sub_of(kh) != part) continue;
                 uint64_t rows = 0, cnt = 0, isum = 0, mn = ~0ull, mx = 0;
                 double dsum = 0.0;
@@ -1229,7 +1248,7 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase2_owned(GView g, uint32_t fi
                     if (omax) mx = max(mx, (uint64_t)a.p_max[at]);
                 }
                 if (!rows) continue;
-                const int s = claim_from(key, (uint32_t)(kh & g.sub_mask));
+                const int s = claim_from(key, home_in(key, kh));
                 if (s >= 0) add(s, (uint32_t)rows, (uint32_t)cnt, REAL ? (uint64_t)__double_as_longlong(dsum) : isum, mn, mx);
                 else g_set_lost(g);
             }
@@ -1287,9 +1306,13 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase2_owned(GView g, uint32_t fi
             uint32_t free_at = 0;  // bit i: from[i] was seen empty
 #pragma unroll
             for (int i = 0; i < kP2Rows; i++) {
-                const uint64_t h = hash64(key[i]);
-                home[i] = (uint32_t)(h & g.sub_mask) | ((uint32_t)(sub_of(h) != part) << 31);
+                const uint64_t h = place(key[i]);
+                home[i] = home_in(key[i], h) | ((uint32_t)(sub_of(h) != part) << 31);
             }
+            if constexpr (IDS) {
+#pragma unroll
+                for (int i = 0; i < kP2Rows; i++) hit[i] = (int)(home[i] & 0x7fffffffu);
+            } else
 #pragma unroll
             for (int i = 0; i < kP2Rows; i++) {
                 const uint32_t b0 = home[i] & (S - 2);
@@ -1350,7 +1373,7 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase2_owned(GView g, uint32_t fi
             const uint32_t s = s0 + u * bd;
             if (s >= S) continue;
             const int64_t gs = base + s;
-            g.keys[gs] = okey[s];
+            if (!IDS) g.keys[gs] = okey[s];
             if (r[u]) g.cntall[gs] = gall[u] + r[u];
             if (!c[u]) continue;
             g.cnt[gs] = gcnt[u] + c[u];
@@ -1367,7 +1390,7 @@ __global__ void __launch_bounds__(kBlock) k_tp_phase2_owned(GView g, uint32_t fi
     }
     // NULL key and key == kEmpty: side slots, summed over the phase-1 workgroups (a strided
     // share per thread, then a sum per wavefront added with device atomics)
-    if (part == 0) {
+    if (!IDS && part == 0) {
         for (int side = 0; side < 2; side++) {
             uint64_t rows = 0, cnt = 0, isum = 0, mn = ~0ull, mx = 0;
             double dsum = 0.0;
@@ -1428,7 +1451,7 @@ int launch_sample(TwoPhaseBufs& b, const KeySpec& ks, const KeyCols& kc, const v
                   int64_t n, int64_t nsamples, int64_t stride, uint64_t smask, hipStream_t s) {
     k_tp_sample<VT, MODE><<<grid_cap(nsamples, 1024, device_info().cus), kSampleBlock, 0, s>>>(
         ks, kc, (const VT*)vals, vnull, mask, ps, vpred, n, stride, nsamples, b.sample_keys,
-        b.sample_cnt, smask);
+        b.sample_cnt, smask, b.id_shift);
     QK_HIP(hipGetLastError());
     return QK_SUCCESS;
 }
@@ -1467,6 +1490,7 @@ P1Args p1_args(const TwoPhaseBufs& b) {
     a.r_count = b.r_count;
     a.zero = b.zero_word;
     a.part_shift = rec_shift_of(b.P);
+    a.id_shift = b.id_shift;
     a.accumulate = b.pending_rows > 0 ? 1 : 0;
     return a;
 }
@@ -1549,7 +1573,9 @@ int launch_p2(TwoPhaseBufs& b, const GView& g, uint32_t fields, hipStream_t s) {
     a.r_rec = b.r_rec;
     a.r_count = b.r_count;
     const bool sum_only = (fields & F_SUM) && !(fields & (F_MIN | F_MAX));
-    const size_t olds = p2o_lds_bytes((int64_t)g.sub_mask + 1, fields);
+    a.id_shift = b.id_shift;
+    const size_t olds = b.id_shift ? p2d_lds_bytes((int64_t)g.sub_mask + 1, fields)
+                                   : p2o_lds_bytes((int64_t)g.sub_mask + 1, fields);
     // sub-tables per partition: a power of two (both counts are), dealt to the dies by eights
     const int64_t F = (int64_t)(g.cap >> g.sub_bits);
     a.split = 0;
@@ -1560,8 +1586,12 @@ int launch_p2(TwoPhaseBufs& b, const GView& g, uint32_t fields, hipStream_t s) {
     if (((int64_t)b.P << a.split) == F && split_ok &&
         olds <= std::min<size_t>(device_info().lds_per_block, 160 * 1024)) {
         // the sub-tables fit the LDS: each workgroup folds into its own sub-table directly
-        if (sum_only) k_tp_phase2_owned<VT, kFieldsSum><<<(int)F, b.block, olds, s>>>(g, fields, a);
-        else k_tp_phase2_owned<VT, kFieldsAny><<<(int)F, b.block, olds, s>>>(g, fields, a);
+        if (b.id_shift && sum_only) k_tp_phase2_owned<VT, kFieldsSum, true><<<(int)F, b.block, olds, s>>>(g, fields, a);
+        else if (b.id_shift) k_tp_phase2_owned<VT, kFieldsAny, true><<<(int)F, b.block, olds, s>>>(g, fields, a);
+        else if (sum_only) k_tp_phase2_owned<VT, kFieldsSum, false><<<(int)F, b.block, olds, s>>>(g, fields, a);
+        else k_tp_phase2_owned<VT, kFieldsAny, false><<<(int)F, b.block, olds, s>>>(g, fields, a);
+    } else if (b.id_shift) {
+        return fail(QK_ERROR, "group by: the slot ranges of a multi-word table do not fit the LDS");
     } else if (sum_only) {
         k_tp_phase2<VT, kFieldsSum><<<b.P, b.block, p2_lds_bytes(b.H2, b.W, fields), s>>>(g, fields, a);
     } else {
@@ -1582,11 +1612,12 @@ void twophase_free(TwoPhaseBufs& b) {
     void* ptrs[] = {b.heavy_keys, b.heavy_cnt, b.cand_cnt, b.heavy_meta, b.sample_keys, b.sample_cnt, b.hist, b.cand,
                     b.p1_image, b.p1_slot,
                     b.p_cnt, b.p_rows, b.p_sum, b.p_min, b.p_max, b.r_rec, b.r_count,
-                    b.zero_word, b.gview};
+                    b.zero_word, b.gview, b.ids};
     for (void* p : ptrs)
         if (p) pool_free(p);
     TwoPhaseBufs fresh;
-    fresh.defer_rows = b.defer_rows;  // a setting, not a buffer
+    fresh.defer_rows = b.defer_rows;  // settings, not buffers
+    fresh.id_shift = b.id_shift;
     b = fresh;
 }
 
@@ -1670,6 +1701,7 @@ int twophase_prepare(TwoPhaseBufs& b, int32_t parts, uint32_t fields, int32_t va
     A((void**)&b.r_count, (size_t)b.W * parts * 4);
     A((void**)&b.zero_word, 64);
     A((void**)&b.gview, sizeof(GView));
+    if (b.id_shift) A((void**)&b.ids, (size_t)n * 4);
     if (st != QK_SUCCESS) {
         twophase_free(b);
         return st;
@@ -1679,7 +1711,7 @@ int twophase_prepare(TwoPhaseBufs& b, int32_t parts, uint32_t fields, int32_t va
     QK_HIP(hipMemsetAsync(b.zero_word, 0, 64, s));
     // the image of the empty heavy set
     k_tp_order<<<1, 1024, (size_t)b.H1 * 8 + (size_t)b.kmax * 12, s>>>(
-        b.cand, b.cand_cnt, b.kmax, b.P, rec_shift_of(b.P), b.heavy_meta, b.heavy_keys, b.heavy_cnt, b.H1,
+        b.cand, b.cand_cnt, b.kmax, b.P, rec_shift_of(b.P), b.id_shift, b.heavy_meta, b.heavy_keys, b.heavy_cnt, b.H1,
         b.p1_image, b.p1_slot);
     QK_HIP(hipGetLastError());
     b.heavy_ready = false;
@@ -1713,7 +1745,7 @@ int twophase_sample(TwoPhaseBufs& b, const GView& g, const KeySpec& ks, const Ke
     k_tp_collect<<<kCollectGrid, kCollectBlock, 0, s>>>(b.sample_keys, b.sample_cnt, (uint64_t)sslots,
                                                                b.kmax, b.heavy_meta, b.cand, b.cand_cnt);
     k_tp_order<<<1, 1024, (size_t)b.H1 * 8 + (size_t)b.kmax * 12, s>>>(
-        b.cand, b.cand_cnt, b.kmax, b.P, rec_shift_of(b.P), b.heavy_meta, b.heavy_keys, b.heavy_cnt, b.H1,
+        b.cand, b.cand_cnt, b.kmax, b.P, rec_shift_of(b.P), b.id_shift, b.heavy_meta, b.heavy_keys, b.heavy_cnt, b.H1,
         b.p1_image, b.p1_slot);
     QK_HIP(hipGetLastError());
     b.heavy_ready = true;

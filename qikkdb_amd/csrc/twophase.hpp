@@ -9,6 +9,11 @@
 // the merge needs no atomics.  Rows that do not fit (NULL values, full regions) take the
 // atomic path in phase 1.
 //
+// Multi-word keys take the same two phases over their slots: a kernel first finds (or claims) each row's
+// slot in the global table and writes it as a 32-bit id (groupby.hip), and the phases then run on the
+// ids, with id << id_shift in the place of the key's hash, so that a partition is a range of slots and
+// phase 2 adds into them without looking anything up.  An id of -1 marks a row that the WHERE drops.
+//
 // Phase 2 may be deferred over several blocks: phase 1 then appends to the regions and adds
 // to the heavy partials, and one phase 2 merges all of them, so the global table is walked
 // once per query instead of once per block.  Whatever reads the table flushes first.
@@ -28,6 +33,8 @@ struct TwoPhaseBufs {
     int32_t H2 = 0;         // phase-2 LDS hash slots
     int32_t block = 1024;   // threads per workgroup (both phases)
     int32_t sample_bits = 18;
+    int32_t id_shift = 0;   // 0: hashed keys; else the keys are slot ids (64 - log2 of the table's slots)
+    int32_t* ids = nullptr; // [block_alloc] the block's slot ids
     int64_t rows_alloc = 0;   // rows the regions were sized for (several blocks when deferring)
     int64_t block_alloc = 0;  // largest block the buffers were sized for
     int64_t defer_rows = -1;  // rows phase 2 may be deferred over: -1 default, 0 never
@@ -72,6 +79,10 @@ __host__ __device__ inline int owned_slot_bytes(uint32_t fields) {
 }
 __host__ __device__ inline size_t p2o_lds_bytes(int64_t S, uint32_t fields) {
     return (size_t)S * (size_t)owned_slot_bytes(fields);
+}
+// The same for slot ids, which need no keys.
+__host__ __device__ inline size_t p2d_lds_bytes(int64_t S, uint32_t fields) {
+    return (size_t)S * (size_t)(owned_slot_bytes(fields) - 8);
 }
 
 // Phase 1 writes cold rows to at most kMaxRecParts partitions (the top bits of the key hash).

@@ -83,3 +83,34 @@ def test_wide_composite_keys(cols, groups, n):
     vals = rng.integers(-10**9, 10**9, n)
     check(ALL, keys, vals, False, key_nulls=kn, value_nulls=rng.random(n) < 0.05,
           capacity=max(64, 40 * groups), block=1 << 18)
+
+
+@pytest.mark.parametrize("flags", [0, qk.GB_ASYNC])
+@pytest.mark.parametrize("capacity", [64, 5000, 300_000, 3_000_000])
+@pytest.mark.parametrize("form", ["plain", "mask", "value_range", "other_column", "mixed"])
+def test_wide_keys_two_phase(form, capacity, flags):
+    """Wide keys through the two phases over their slots, forced at every block size: one slot range up
+    to several per partition, NULL keys and values, deferred and immediate merges, and every form of WHERE
+    (rows it drops must not create groups)."""
+    rng = np.random.default_rng(capacity + len(form))
+    n, groups = 300_007, min(capacity // 2, 40_000)
+    code = np.where(rng.random(n) < 0.5, rng.integers(0, 1 + groups // 50, n), rng.integers(0, groups, n))
+    keys = [(code % 211 - 100).astype(np.int32), (code // 211).astype(np.int64)]
+    kn = [rng.random(n) < 0.01, None] if capacity > 64 else None
+    if kn is None:
+        keys[0] = keys[0] * 0
+    vals, vn = rng.lognormal(0, 1, n), rng.random(n) < 0.05
+    other = rng.integers(0, 100, n).astype(np.int32)
+    kw = {"extra_cols": {"other": (other, rng.random(n) < 0.05)}}
+    if form == "mask":
+        kw = {"mask": (rng.random(n) < 0.3).astype(np.int8)}
+    elif form == "value_range":
+        kw["where"] = [Where(qk.GREATER, "value", 0.5, qk.DOUBLE), Where(qk.LESS, "value", 4.0, qk.DOUBLE)]
+    elif form == "other_column":
+        kw["where"] = [Where(qk.LESS, "other", 40, qk.INT)]
+    elif form == "mixed":
+        kw["where"] = [Where(qk.NOT_EQUAL, "other", 7, qk.INT), Where(qk.GREATER, "value", 0.25, qk.DOUBLE)]
+    stats = {}
+    check(ALL, keys, vals, True, key_nulls=kn, value_nulls=vn, capacity=capacity, flags=flags, path=1,
+          block=70_016, stats=stats, **kw)
+    assert stats["path"] == 1 and stats["p1_form"] == 1
