@@ -66,57 +66,57 @@ __global__ void __launch_bounds__(1024) k_gb_rows(GView g, KeySpec ks, KeyCols k
     const int64_t bd = blockDim.x;
     const int64_t tile_rows = bd * kSteps;
     const int64_t ntiles = (n + tile_rows - 1) / tile_rows;
-    struct Tile {
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        // rows past the end read the last row and are dropped: the loads are unconditional, so those of
+        // a tile are all in flight together
         uint64_t key[kSteps][KW];
-        bool kn[kSteps], vn[kSteps], keep[kSteps], cn[kSteps];
-        int64_t cv[kSteps];
-        typename std::conditional<HAS_V, VT, int>::type val[kSteps];
-    };
-    // rows past the end read the last row and are dropped: the loads are unconditional, so those of a
-    // tile are all in flight together
-    auto row_of = [&](int64_t tile, int k) { return tile * tile_rows + k * bd + threadIdx.x; };
-    auto load = [&](int64_t tile, Tile& T) {
         int64_t r[kSteps];
-#pragma unroll
-        for (int k = 0; k < kSteps; k++) r[k] = min(row_of(tile, k), n - 1);
-        load_keys<KW, kSteps>(ks, kc, r, T.key, T.kn);
+        bool kn[kSteps], act[kSteps], vn[kSteps];
+        typename std::conditional<HAS_V, VT, int>::type val[kSteps];
 #pragma unroll
         for (int k = 0; k < kSteps; k++) {
-            T.val[k] = {};
-            if constexpr (HAS_V) T.val[k] = vals[r[k]];
+            const int64_t row = tile * tile_rows + k * bd + threadIdx.x;
+            act[k] = row < n;
+            r[k] = min(row, n - 1);
+        }
+        load_keys<KW, kSteps>(ks, kc, r, key, kn);
+#pragma unroll
+        for (int k = 0; k < kSteps; k++) {
+            val[k] = {};
+            if constexpr (HAS_V) val[k] = vals[r[k]];
         }
 #pragma unroll
-        for (int k = 0; k < kSteps; k++) T.vn[k] = vnull && null_bit(vnull, r[k]);
+        for (int k = 0; k < kSteps; k++) vn[k] = vnull && null_bit(vnull, r[k]);
+        if (MODE == 1) {
 #pragma unroll
-        for (int k = 0; k < kSteps; k++) {
-            T.keep[k] = MODE == 1 ? mask[r[k]] != 0 : true;
-            T.cv[k] = 0;
-            T.cn[k] = false;
-            if (MODE == 4) {
-                T.cv[k] = range_col(preds, r[k]);
-                T.cn[k] = preds.rnull && null_bit(preds.rnull, r[k]);
-            }
+            for (int k = 0; k < kSteps; k++) act[k] = act[k] & (mask[r[k]] != 0);
         }
-    };
-    auto process = [&](int64_t tile, const Tile& T) {
-        bool act[kSteps];
+        if (MODE == 4) {
+            int64_t cv[kSteps];
 #pragma unroll
-        for (int k = 0; k < kSteps; k++) {
-            const int64_t r = row_of(tile, k);
-            act[k] = (r < n) & T.keep[k];
-            if (MODE == 4) act[k] = act[k] & !T.cn[k] & col_in_range(preds, T.cv[k]);
-            if constexpr (MODE == 3 && HAS_V) act[k] = act[k] & !T.vn[k] & in_range<VT>(preds.vr, T.val[k]);
-            if (MODE == 2 && act[k]) {
+            for (int k = 0; k < kSteps; k++) cv[k] = range_col(preds, r[k]);
+#pragma unroll
+            for (int k = 0; k < kSteps; k++)
+                act[k] = act[k] & !(preds.rnull && null_bit(preds.rnull, r[k])) & col_in_range(preds, cv[k]);
+        }
+        if constexpr (MODE == 3 && HAS_V) {
+#pragma unroll
+            for (int k = 0; k < kSteps; k++) act[k] = act[k] & !vn[k] & in_range<VT>(preds.vr, val[k]);
+        }
+        if (MODE == 2) {
+#pragma unroll
+            for (int k = 0; k < kSteps; k++) {
+                if (!act[k]) continue;
                 bool pass = true;
                 for (int p = 0; p < preds.n && pass; p++) {
                     const qk_predicate& q = preds.p[p];
                     if constexpr (HAS_V) {
                         if ((vpred >> p) & 1u) {
-                            pass = !T.vn[k] && pred_on_value(q, T.val[k], r);
+                            pass = !vn[k] && pred_on_value(q, val[k], r[k]);
                             continue;
                         }
                     }
-                    pass = eval_pred(q, r);
+                    pass = eval_pred(q, r[k]);
                 }
                 act[k] = pass;
             }
@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(1024) k_gb_rows(GView g, KeySpec ks, KeyCols k
         if constexpr (KW > 1) {
 #pragma unroll
             for (int k = 0; k < kSteps; k++) {
-                home[k] = home_of(g, key_hash<KW>(T.key[k]));
+                home[k] = home_of(g, key_hash<KW>(key[k]));
                 tail[k] = g_key_tail<KW>(g, home[k]);
             }
         }
@@ -135,20 +135,20 @@ __global__ void __launch_bounds__(1024) k_gb_rows(GView g, KeySpec ks, KeyCols k
         for (int k = 0; k < kSteps; k++) {
             if (!act[k]) continue;
             Part p;
-            if constexpr (HAS_V) p = row_part<VT>(T.val[k], T.vn[k]); else p = row_part<NoValue>(NoValue{}, T.vn[k]);
+            if constexpr (HAS_V) p = row_part<VT>(val[k], vn[k]); else p = row_part<NoValue>(NoValue{}, vn[k]);
             bool is_new = false;
             if constexpr (KW == 1) {
-                const uint64_t h = hash64(T.key[k][0]);
-                int ls = use_lds ? lds_find(t, T.key[k][0], T.kn[k], h) : -1;
+                const uint64_t h = hash64(key[k][0]);
+                int ls = use_lds ? lds_find(t, key[k][0], kn[k], h) : -1;
                 if (ls >= 0) {
                     lds_accum<REAL>(t, (ls << rbits) | copy, p, fields);
                 } else {
-                    const int64_t gs = g_slot1(g, T.key[k][0], T.kn[k], h, &is_new);
+                    const int64_t gs = g_slot1(g, key[k][0], kn[k], h, &is_new);
                     if (gs >= 0) g_accum_atomic(g, gs, p, fields); else g_set_lost(g);
                 }
             } else {
-                int64_t gs = g_find_cached<KW>(g, T.key[k], home[k], tail[k]);
-                if (gs < 0) gs = g_slotN<KW>(g, T.key[k], key_hash<KW>(T.key[k]), &is_new);
+                int64_t gs = g_find_cached<KW>(g, key[k], home[k], tail[k]);
+                if (gs < 0) gs = g_slotN<KW>(g, key[k], key_hash<KW>(key[k]), &is_new);
                 if (gs < 0) {
                     g_set_lost(g);
                 } else {
@@ -158,27 +158,6 @@ __global__ void __launch_bounds__(1024) k_gb_rows(GView g, KeySpec ks, KeyCols k
                 }
             }
             if (is_new) atomicAdd(&s_new, 1u);
-        }
-    };
-    int64_t tile = blockIdx.x;
-    if constexpr (KW == 1 && MODE != 2) {
-        // the next tile's loads are issued before this tile is aggregated (two register sets)
-        Tile A, B;
-        if (tile < ntiles) load(tile, A);
-        while (tile < ntiles) {
-            load(tile + gridDim.x, B);
-            process(tile, A);
-            tile += gridDim.x;
-            if (tile >= ntiles) break;
-            load(tile + gridDim.x, A);
-            process(tile, B);
-            tile += gridDim.x;
-        }
-    } else {
-        for (; tile < ntiles; tile += gridDim.x) {
-            Tile A;
-            load(tile, A);
-            process(tile, A);
         }
     }
 
@@ -622,7 +601,7 @@ int launch_rows_t(const GView& g, const KeySpec& ks, const KeyCols& kc, const vo
     const int64_t tile_rows = (int64_t)block * kSteps;
     const int64_t ntiles = (n + tile_rows - 1) / tile_rows;
     int64_t grid = (int64_t)device_info().cus * occ;
-    if (L.all) grid = std::min<int64_t>({grid, kMaxPartials, (n + L.min_rows - 1) / L.min_rows});
+    if (L.all) grid = std::min(grid, L.wgs_for(n));
     if (grid > ntiles) grid = ntiles;
     if (grid < 1) grid = 1;
     const Partials part = L.for_wgs(grid);

@@ -142,8 +142,8 @@ __device__ __forceinline__ Part lds_fold(const Lds& t, int s, int first) {
 }
 
 // Merges one LDS entry (its key or, of a multi-word key, its global slot; side 0 and 1: the entries of
-// the NULL key and of the key equal to kEmpty) into the global table.
-template <int KW>
+// the NULL key and of the key equal to kEmpty) into the global table.  READ as in g_accum_atomic.
+template <int KW, bool READ>
 __device__ __forceinline__ void add_entry(const GView& g, uint64_t k, int side, const Part& p, uint32_t fields,
                                           unsigned int* s_new) {
     bool is_new = false;
@@ -158,7 +158,7 @@ __device__ __forceinline__ void add_entry(const GView& g, uint64_t k, int side, 
         gs = g_slot1(g, k, false, hash64(k), &is_new);
     }
     if (is_new) atomicAdd(s_new, 1u);
-    if (gs >= 0) g_accum_atomic<false>(g, gs, p, fields); else g_set_lost(g);
+    if (gs >= 0) g_accum_atomic<READ>(g, gs, p, fields); else g_set_lost(g);
 }
 
 // The workgroups' LDS tables in global memory: arrays [workgroup][H + 2] of keys (kEmpty: no entry)
@@ -186,7 +186,7 @@ __device__ __forceinline__ void lds_flush(const Lds& t, const GView& g, const Pa
                 if (t.mx) out.mx[at] = p.mx;
             }
         } else if (used) {
-            add_entry<KW>(g, k, s - t.H, lds_fold<REAL>(t, s, threadIdx.x), fields, s_new);
+            add_entry<KW, true>(g, k, s - t.H, lds_fold<REAL>(t, s, threadIdx.x), fields, s_new);
         }
     }
 }
@@ -205,6 +205,12 @@ struct LdsShape {
     int64_t min_rows = 0, keys = 0;
     Partials part{};
 
+    // workgroups for n rows: min_rows each, but no fewer than 64 (82K rows, 651 groups of a wide key: 70 us
+    // in 10 workgroups)
+    int64_t wgs_for(int64_t n) const {
+        const int64_t w = (n + min_rows - 1) / min_rows;
+        return w < 64 ? 64 : (w > kMaxPartials ? kMaxPartials : w);
+    }
     Partials for_wgs(int64_t wgs) const { return wgs * keys > kDirectEntries ? part : Partials{}; }
 };
 

@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(kFoldBlock) k_gb_fold(GView g, Partials in, in
             if (k == kEmpty) return;
             const int ls = lds_find(t, side == 1 ? kEmpty : k, side == 0, hash64(k));
             if (ls >= 0) lds_accum<REAL>(t, ls, p, fields);
-            else add_entry<KW>(g, k, side, p, fields, &s_new);
+            else add_entry<KW, false>(g, k, side, p, fields, &s_new);
         };
         // kFoldBatch tables' entries at a time, key and states loaded together (an empty entry's states
         // are whatever memory holds, and are dropped)
@@ -137,7 +137,7 @@ __global__ void __launch_bounds__(kFoldBlock) k_gb_fold(GView g, Partials in, in
     for (int e = threadIdx.x; e < kFoldH + 2; e += blockDim.x) {
         const uint64_t k = t.key[e];
         if (e < kFoldH ? k == kEmpty : k == 0ull) continue;
-        add_entry<KW>(g, k, e - kFoldH, lds_fold<REAL>(t, e, 0), fields, &s_new);
+        add_entry<KW, false>(g, k, e - kFoldH, lds_fold<REAL>(t, e, 0), fields, &s_new);
     }
     __syncthreads();
     if (threadIdx.x == 0) g_count_new(g, s_new);
@@ -156,7 +156,7 @@ int launch_small(const GView& g, const KeyCols& kc, const void* vals, const uint
     QK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, kSmallBlock, lds));
     if (occ < 1) return fail(QK_ERROR, "group by: small-table launch (LDS %zu B) does not fit", lds);
     const int64_t grid = std::max<int64_t>(
-        1, std::min<int64_t>({(int64_t)device_info().cus * occ, kMaxPartials, (n + L.min_rows - 1) / L.min_rows,
+        1, std::min<int64_t>({(int64_t)device_info().cus * occ, L.wgs_for(n),
                               (n + kSChunk * (kSmallBlock / 64) - 1) / (kSChunk * (kSmallBlock / 64))}));
     const Partials part = L.for_wgs(grid);
     kern<<<(unsigned)grid, kSmallBlock, lds, s>>>(g, kc, (const VT*)vals, vnull, ps, (int32_t)n, fields, L.H, hshift,
