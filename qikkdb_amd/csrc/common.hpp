@@ -61,8 +61,27 @@ struct Scratch {
 // counts.
 int stream_scratch(hipStream_t s, size_t bytes, Scratch** out, int kind = 0);
 
-// Small pinned host buffer per thread for count read-backs.
-int pinned_host(size_t bytes, void** out);
+// Up to kBackSegs pieces of device memory (whole 32-bit words, kBackBytes in all) to the host, after the
+// work queued on the stream; *out: their bytes one after the other, valid until the thread's next call.
+// A kernel writes them and a ticket to pinned memory and the host watches the ticket: a copy and a
+// stream synchronisation take 15-20 us more than the work itself, this about 6.  read_back_sum: the sum
+// of n int32 counts.
+constexpr int kBackSegs = 3;
+constexpr size_t kBackBytes = 1024;
+struct BackSeg {
+    const void* src;
+    uint32_t bytes;
+};
+int read_back(hipStream_t s, const BackSeg* segs, int nsegs, const void** out);
+int read_back_sum(hipStream_t s, const int32_t* counts, int32_t n, int64_t* out);
+template <typename T>
+inline int read_back_one(hipStream_t s, const T* src, T* out) {
+    const BackSeg seg{src, sizeof(T)};
+    const void* p = nullptr;
+    const int st = read_back(s, &seg, 1, &p);
+    if (st == QK_SUCCESS) *out = *(const T*)p;
+    return st;
+}
 
 // Whether a batch engine may keep a ts-ordered copy of its table (batch.hip; on by default), and the
 // device memory the copy takes (0: the table has none).

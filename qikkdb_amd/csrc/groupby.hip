@@ -839,12 +839,7 @@ int flush_pending(qk_groupby_s* h, hipStream_t s) {
 }
 
 int read_counters(qk_groupby_s* h, hipStream_t s, TableCounters* out) {
-    void* hb = nullptr;
-    QK_TRY(pinned_host(sizeof(TableCounters), &hb));
-    QK_HIP(hipMemcpyAsync(hb, h->ctr, sizeof(TableCounters), hipMemcpyDeviceToHost, s));
-    QK_HIP(hipStreamSynchronize(s));
-    memcpy(out, hb, sizeof(TableCounters));
-    return QK_SUCCESS;
+    return read_back_one(s, h->ctr, out);
 }
 
 // Read and clear the latched error (ErrorFlagSwapper::Swap, ErrorFlagSwapper.h:32-48).
@@ -1395,12 +1390,8 @@ int qk_gb_group_count(qk_groupby h, int64_t* out, void* stream) {
     QK_TRY(read_counters(h, s, &c));
     uint64_t side = 0;
     if (h->ks.kw == 1) {
-        void* hb = nullptr;
-        QK_TRY(pinned_host(8, &hb));
-        QK_HIP(hipMemcpyAsync(hb, h->keys + h->cap, 8, hipMemcpyDeviceToHost, s));
-        QK_HIP(hipStreamSynchronize(s));
-        uint64_t w;
-        memcpy(&w, hb, 8);
+        uint64_t w = 0;
+        QK_TRY(read_back_one(s, h->keys + h->cap, &w));
         side = w != 0 ? 1 : 0;  // the NULL group
     }
     *out = (int64_t)(c.nkeys + side);
@@ -1436,17 +1427,13 @@ int get_results_impl(qk_groupby h, int32_t naggs, const int32_t* aggs, const int
     TableCounters c;
     bool null_group = false;
     {
-        void* hb = nullptr;
-        QK_TRY(pinned_host(64, &hb));
-        QK_HIP(hipMemcpyAsync(hb, h->ctr, sizeof(TableCounters), hipMemcpyDeviceToHost, s));
-        if (h->ks.kw == 1)
-            QK_HIP(hipMemcpyAsync((char*)hb + 32, h->keys + h->cap, 8, hipMemcpyDeviceToHost, s));
-        QK_HIP(hipStreamSynchronize(s));
-        static_assert(sizeof(TableCounters) <= 32, "counters and slot word share the staging buffer");
+        const BackSeg segs[2] = {{h->ctr, sizeof(TableCounters)}, {h->keys + h->cap, 8}};
+        const void* hb = nullptr;
+        QK_TRY(read_back(s, segs, h->ks.kw == 1 ? 2 : 1, &hb));
         memcpy(&c, hb, sizeof(TableCounters));
         if (h->ks.kw == 1) {
             uint64_t w;
-            memcpy(&w, (char*)hb + 32, 8);
+            memcpy(&w, (const char*)hb + sizeof(TableCounters), 8);
             null_group = w != 0;
         }
     }
@@ -1531,15 +1518,7 @@ int get_results_impl(qk_groupby h, int32_t naggs, const int32_t* aggs, const int
         e = hipGetLastError();
     }
     int32_t written = 0;
-    if (e == hipSuccess) {
-        void* hb = nullptr;
-        st = pinned_host(8, &hb);
-        if (st == QK_SUCCESS) {
-            e = hipMemcpyAsync(hb, total, 4, hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipStreamSynchronize(s);
-            if (e == hipSuccess) written = *(int32_t*)hb;
-        }
-    }
+    if (e == hipSuccess) st = read_back_one(s, total, &written);
     if (e != hipSuccess || st != QK_SUCCESS) {
         cleanup();
         return st != QK_SUCCESS ? st : fail(QK_RUNTIME_ERROR, "qk_gb_get_results: %s", hipGetErrorString(e));

@@ -454,21 +454,12 @@ struct Compaction {
 
     // After the first pass: scans the counts and reads the number of kept rows back.
     int count(hipStream_t s) {
-        void* h = nullptr;
-        if (self) {
-            QK_TRY(pinned_host((size_t)tiles * 4, &h));
-            QK_HIP(hipMemcpyAsync(h, counts, (size_t)tiles * 4, hipMemcpyDeviceToHost, s));
-            QK_HIP(hipStreamSynchronize(s));
-            kept = 0;
-            for (int64_t i = 0; i < tiles; i++) kept += ((const int32_t*)h)[i];
-            return QK_SUCCESS;
-        }
+        if (self) return read_back_sum(s, counts, (int32_t)tiles, &kept);
         k_scan_counts<<<1, 1024, 0, s>>>(counts, tiles, total);
         QK_HIP(hipGetLastError());
-        QK_TRY(pinned_host(8, &h));
-        QK_HIP(hipMemcpyAsync(h, total, 4, hipMemcpyDeviceToHost, s));
-        QK_HIP(hipStreamSynchronize(s));
-        kept = *(const int32_t*)h;
+        int32_t all = 0;
+        QK_TRY(read_back_one(s, total, &all));
+        kept = all;
         return QK_SUCCESS;
     }
 
@@ -619,12 +610,7 @@ int qk_mask_sum(const int8_t* mask, int32_t n, int64_t* out_host, void* stream) 
     QK_HIP(hipMemsetAsync(ctr, 0, 8, s));
     k_mask_reduce<<<grid_stride_blocks(((int64_t)n + 15) / 16, 256), 256, 0, s>>>(mask, n, ctr);
     QK_HIP(hipGetLastError());
-    void* h = nullptr;
-    QK_TRY(pinned_host(8, &h));
-    QK_HIP(hipMemcpyAsync(h, ctr, 8, hipMemcpyDeviceToHost, s));
-    QK_HIP(hipStreamSynchronize(s));
-    *out_host = *(int64_t*)h;
-    return QK_SUCCESS;
+    return read_back_one(s, (const int64_t*)ctr, out_host);
 }
 
 int qk_reconstruct_col_keep(int32_t elem_size, const void* in, const int8_t* mask, int32_t n,

@@ -197,18 +197,110 @@ int stream_scratch(hipStream_t s, size_t bytes, Scratch** out, int kind) {
     return QK_SUCCESS;
 }
 
-int pinned_host(size_t bytes, void** out) {
-    static thread_local void* buf = nullptr;
-    static thread_local size_t cap = 0;
-    if (cap < bytes) {
-        if (buf) (void)hipHostFree(buf);
-        buf = nullptr;
-        size_t nb = 4096;
-        while (nb < bytes) nb <<= 1;
-        QK_HIP(hipHostMalloc(&buf, nb, hipHostMallocDefault));
-        cap = nb;
+// ---- read-backs ----------------------------------------------------------------------------
+
+namespace {
+
+// One thread's pinned page: the ticket of the last read-back written, then its bytes.
+struct BackPage {
+    uint64_t ticket;
+    char pad[56];
+    uint32_t words[kBackBytes / 4];
+};
+struct BackSegs {
+    int32_t n;
+    BackSeg s[kBackSegs];
+};
+
+__device__ __forceinline__ void back_publish(BackPage* page, uint64_t ticket) {
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(&page->ticket, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void __launch_bounds__(256) k_read_back(BackSegs segs, BackPage* page, uint64_t ticket) {
+    uint32_t at = 0;
+    for (int i = 0; i < segs.n; i++) {
+        const uint32_t words = segs.s[i].bytes / 4;
+        for (uint32_t w = threadIdx.x; w < words; w += blockDim.x) page->words[at + w] = ((const uint32_t*)segs.s[i].src)[w];
+        at += words;
     }
-    *out = buf;
+    back_publish(page, ticket);
+}
+
+__global__ void __launch_bounds__(256) k_read_back_sum(const int32_t* __restrict__ counts, int32_t n, BackPage* page,
+                                                       uint64_t ticket) {
+    __shared__ int64_t s_part[4];
+    int64_t v = 0;
+    for (int32_t i = threadIdx.x; i < n; i += blockDim.x) v += counts[i];
+    v = wave_sum64(v);
+    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) *(int64_t*)page->words = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+    back_publish(page, ticket);
+}
+
+// The thread's page, given back when the thread ends.
+struct BackPageOwner {
+    BackPage* page = nullptr;
+    uint64_t ticket = 0;
+    ~BackPageOwner() {
+        if (page) (void)hipHostFree(page);
+    }
+};
+
+int back_page(BackPageOwner** out) {
+    static thread_local BackPageOwner o;
+    if (!o.page) {
+        void* p = nullptr;
+        QK_HIP(hipHostMalloc(&p, sizeof(BackPage), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
+        memset(p, 0, sizeof(BackPage));
+        o.page = (BackPage*)p;
+    }
+    *out = &o;
+    return QK_SUCCESS;
+}
+
+// Waits for the page's ticket: by watching it for a while (most calls wait a few microseconds), then by
+// synchronising the stream, which also reports an error of the queued work.
+int back_wait(const BackPageOwner& o, hipStream_t s) {
+    const uint64_t* t = &o.page->ticket;
+    for (int i = 0; i < 20000; i++) {
+        if (__atomic_load_n(t, __ATOMIC_ACQUIRE) == o.ticket) return QK_SUCCESS;
+        __builtin_ia32_pause();
+    }
+    QK_HIP(hipStreamSynchronize(s));
+    if (__atomic_load_n(t, __ATOMIC_ACQUIRE) != o.ticket)
+        return fail(QK_RUNTIME_ERROR, "a read-back ended without its result");
+    return QK_SUCCESS;
+}
+
+}  // namespace
+
+int read_back(hipStream_t s, const BackSeg* segs, int nsegs, const void** out) {
+    BackSegs bs{};
+    size_t bytes = 0;
+    for (int i = 0; i < nsegs && i < kBackSegs; i++) {
+        bs.s[bs.n++] = segs[i];
+        bytes += segs[i].bytes;
+    }
+    if (nsegs > kBackSegs || bytes > kBackBytes) return fail(QK_RUNTIME_ERROR, "read-back of %zu bytes", bytes);
+    BackPageOwner* o = nullptr;
+    QK_TRY(back_page(&o));
+    k_read_back<<<1, 256, 0, s>>>(bs, o->page, ++o->ticket);
+    QK_HIP(hipGetLastError());
+    QK_TRY(back_wait(*o, s));
+    *out = o->page->words;
+    return QK_SUCCESS;
+}
+
+int read_back_sum(hipStream_t s, const int32_t* counts, int32_t n, int64_t* out) {
+    BackPageOwner* o = nullptr;
+    QK_TRY(back_page(&o));
+    k_read_back_sum<<<1, 256, 0, s>>>(counts, n, o->page, ++o->ticket);
+    QK_HIP(hipGetLastError());
+    QK_TRY(back_wait(*o, s));
+    memcpy(out, o->page->words, 8);
     return QK_SUCCESS;
 }
 

@@ -286,7 +286,6 @@ struct qk_gbs_s {
     int64_t slot_cap = 0;
     unsigned int* counters = nullptr;
     unsigned long long* arena_used = nullptr;
-    void* host = nullptr;      // pinned: counters and block totals read back
 };
 
 namespace {
@@ -308,7 +307,6 @@ void gbs_free(qk_gbs_s* h) {
     for (void* p : {(void*)h->slots, (void*)h->off, (void*)h->len, (void*)h->arena, (void*)h->newlist,
                     (void*)h->slot_col, (void*)h->counters})
         if (p) qk::pool_free(p);
-    if (h->host) (void)hipHostFree(h->host);
     if (h->inner) qk_gb_destroy(h->inner);
 }
 
@@ -352,10 +350,8 @@ int gbs_block(qk_gbs_s* h, const char* chars, const int64_t* indices, const uint
     QK_TRY(qk::check_preds(npreds, preds, &ps));
     hipStream_t s = qk::as_stream(stream);
     // bytes of the block: indices[n-1]
-    int64_t* hb = (int64_t*)h->host;
-    QK_HIP(hipMemcpyAsync(hb, indices + n - 1, 8, hipMemcpyDeviceToHost, s));
-    QK_HIP(hipStreamSynchronize(s));
-    const int64_t total = hb[0];
+    int64_t total = 0;
+    QK_TRY(qk::read_back_one(s, indices + n - 1, &total));
     if (total < 0) return qk::fail(QK_ERROR, "string group by: negative string offsets");
     if (total > 0 && !chars) return qk::fail(QK_ERROR, "string group by: null chars");
     QK_TRY(gbs_reserve(h, n, total, s));
@@ -370,10 +366,9 @@ int gbs_block(qk_gbs_s* h, const char* chars, const int64_t* indices, const uint
     k_str_commit<<<grid_for(n), 256, 0, s>>>(d, chars, indices);
     QK_HIP(hipGetLastError());
     h->arena_bound += total;
-    unsigned int* hc = (unsigned int*)((char*)h->host + 16);
-    QK_HIP(hipMemcpyAsync(hc, h->counters, 8, hipMemcpyDeviceToHost, s));
-    QK_HIP(hipStreamSynchronize(s));
-    if (hc[1]) return qk::fail(QK_HASH_TABLE_FULL, "string group by: the string dictionary is full");
+    unsigned int lost = 0;
+    QK_TRY(qk::read_back_one(s, (const unsigned int*)h->counters + 1, &lost));
+    if (lost) return qk::fail(QK_HASH_TABLE_FULL, "string group by: the string dictionary is full");
     const void* kp[1] = {h->slot_col};
     const uint64_t* kn[1] = {key_nulls};
     return qk_gb_process_block_where(h->inner, kp, key_nulls ? kn : nullptr, values, value_nulls, n, npreds, preds,
@@ -410,8 +405,6 @@ int qk_gbs_create(qk_gbs* out, int32_t value_type, int32_t naggs, const int32_t*
     A((void**)&h->len, (size_t)D * 4);
     A((void**)&h->counters, 64);
     if (st == QK_SUCCESS) h->arena_used = (unsigned long long*)(h->counters + 8);
-    if (st == QK_SUCCESS && hipHostMalloc(&h->host, 64, hipHostMallocDefault) != hipSuccess)
-        st = qk::fail(QK_OUT_OF_MEMORY, "string group by: pinned host buffer");
     if (st == QK_SUCCESS) st = qk_gbs_reset(h, nullptr);
     if (st == QK_SUCCESS) st = qk_stream_synchronize(nullptr);
     if (st != QK_SUCCESS) {
@@ -479,11 +472,9 @@ int qk_gbs_get_results(qk_gbs h, char** out_chars, int64_t** out_indices, uint64
         k_scan64_sums<<<(unsigned)nb, kScanThreads, 0, s>>>(lens, g, sums);
         k_scan64_top<<<1, kScanThreads, 0, s>>>(sums, nb);
         k_scan64_apply<<<(unsigned)nb, kScanThreads, 0, s>>>(lens, g, sums);
-        int64_t* hb = (int64_t*)h->host;
-        if (hipMemcpyAsync(hb, lens + g - 1, 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            st = qk::fail(QK_RUNTIME_ERROR, "string group by: reading the result size");
-        if (st == QK_SUCCESS) st = qk::pool_alloc((void**)&chars, (size_t)std::max<int64_t>(hb[0], 1));
+        int64_t total = 0;
+        st = qk::read_back_one(s, lens + g - 1, &total);
+        if (st == QK_SUCCESS) st = qk::pool_alloc((void**)&chars, (size_t)std::max<int64_t>(total, 1));
         if (st == QK_SUCCESS) {
             k_str_gather<<<grid_for(g), 256, 0, s>>>(d, (const int64_t*)keys[0], kn[0], g, lens, chars);
             if (hipGetLastError() != hipSuccess) st = qk::fail(QK_RUNTIME_ERROR, "string group by: gather launch");
