@@ -942,6 +942,14 @@ LdsShape choose_lds(const qk_groupby_s* h) {
     return L;
 }
 
+// Whether the stream is being captured (or cannot say).
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) return false;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Memory for the workgroups' tables, kept with the table.  Without it (no memory left, or a first
 // block under graph capture, where nothing can be allocated) they go straight to the global table;
 // so do those of an asynchronous table's blocks on another stream than the first, which may run
@@ -952,11 +960,7 @@ void partials_for(qk_groupby_s* h, LdsShape* L, hipStream_t s) {
     int arrays = 2;
     for (uint32_t f : {F_CNTALL, F_SUM, F_MIN, F_MAX}) arrays += (h->fields & f) ? 1 : 0;
     if (h->part_words < words) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
-            return;
-        }
+        if (capturing(s)) return;
         if (h->part_buf) {
             // another stream's last block may still use the smaller one
             if (hipDeviceSynchronize() != hipSuccess) return;
@@ -980,6 +984,23 @@ void partials_for(qk_groupby_s* h, LdsShape* L, hipStream_t s) {
     L->part.sum = next(h->fields & F_SUM);
     L->part.mn = next(h->fields & F_MIN);
     L->part.mx = next(h->fields & F_MAX);
+}
+
+// The two phases' buffers for a block of n rows; pending rows are merged first when they must go.
+int prepare_two(qk_groupby_s* h, int32_t n, bool has_values, int32_t vtype, bool defer, hipStream_t s) {
+    TwoPhaseBufs& tp = h->tp;
+    const int32_t id_shift = h->ks.kw > 1 ? 64 - log2_of(h->cap) : 0;
+    if (tp.id_shift != id_shift) {  // the table's first such block, or it has grown (nothing is pending)
+        if (tp.r_rec) {
+            QK_HIP(hipDeviceSynchronize());
+            twophase_free(tp);
+        }
+        tp.id_shift = id_shift;
+    }
+    if (tp.pending_rows > 0 && (twophase_needs_realloc(tp, h->rec_parts, h->value_type, has_values, n, defer) ||
+                                tp.pending_rows + n > tp.rows_alloc || tp.pend_vtype != vtype))
+        QK_TRY(twophase_flush(tp, phase_view(h), h->fields, s));
+    return twophase_prepare(tp, h->rec_parts, h->fields, h->value_type, has_values, n, defer, s);
 }
 
 // The slot ids of a block.  Its first rows go ahead on their own: they bring the frequent keys into the
@@ -1048,30 +1069,24 @@ int process_once(qk_groupby h, int mode, const void* const* keys, const uint64_t
     // a table whose every key fits a workgroup's LDS takes the one-pass kernel at any size
     LdsShape L = choose_lds(h);
     const bool ids = h->ks.kw > 1;
-    const bool two = (ids ? h->id_parts > 0 : twophase_supported(h->ks.kw, h->value_type)) &&
-                     (h->twophase_mode == 1 ||
-                      (h->twophase_mode < 0 && n >= h->twophase_min_rows && !L.all));
+    bool two = (ids ? h->id_parts > 0 : twophase_supported(h->ks.kw, h->value_type)) &&
+               (h->twophase_mode == 1 || (h->twophase_mode < 0 && n >= h->twophase_min_rows && !L.all));
+    // Phase 2 is deferred across blocks only for asynchronous tables: a synchronous table
+    // reports a full table at the block that filled it, as the reference does, and a
+    // growing table grows at the block that filled it.
+    const bool defer = (h->flags & (QK_GB_ASYNC | QK_GB_AUTO_GROW)) == QK_GB_ASYNC && h->tp.defer_rows != 0;
+    // the one-pass kernel needs no memory of its own: it takes a multi-word table's blocks where
+    // the phases' cannot be had (no memory left, or under graph capture)
+    if (two && ids && capturing(s)) two = false;
+    if (two) {
+        const int prepared = prepare_two(h, n, values != nullptr, vtype, defer, s);
+        if (ids && prepared == QK_OUT_OF_MEMORY) two = false;
+        else QK_TRY(prepared);
+    }
     int st;
     if (two) {
-        // Phase 2 is deferred across blocks only for asynchronous tables: a synchronous table
-        // reports a full table at the block that filled it, as the reference does, and a
-        // growing table grows at the block that filled it.
-        const bool defer = (h->flags & (QK_GB_ASYNC | QK_GB_AUTO_GROW)) == QK_GB_ASYNC && h->tp.defer_rows != 0;
         TwoPhaseBufs& tp = h->tp;
         const GView gp = phase_view(h);
-        const int32_t id_shift = ids ? 64 - log2_of(h->cap) : 0;
-        if (tp.id_shift != id_shift) {  // the table's first such block, or it has grown (nothing is pending)
-            if (tp.r_rec) {
-                QK_HIP(hipDeviceSynchronize());
-                twophase_free(tp);
-            }
-            tp.id_shift = id_shift;
-        }
-        if (tp.pending_rows > 0 &&
-            (twophase_needs_realloc(tp, h->rec_parts, h->value_type, values != nullptr, n, defer) ||
-             tp.pending_rows + n > tp.rows_alloc || tp.pend_vtype != vtype))
-            QK_TRY(twophase_flush(tp, gp, h->fields, s));
-        QK_TRY(twophase_prepare(tp, h->rec_parts, h->fields, h->value_type, values != nullptr, n, defer, s));
         // the rows as the phases read them: the block's columns, or its slot ids (the WHERE is done then)
         KeySpec pks = h->ks;
         KeyCols pkc = kc;

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import qikkdb_amd as qk
-from gpu_util import Where, cpu_group_by, gpu_group_by
+from gpu_util import Where, col, cpu_group_by, gpu_group_by
 from helpers import as_map, maps_close
 
 pytestmark = pytest.mark.gpu
@@ -114,3 +114,36 @@ def test_wide_keys_two_phase(form, capacity, flags):
     check(ALL, keys, vals, True, key_nulls=kn, value_nulls=vn, capacity=capacity, flags=flags, path=1,
           block=70_016, stats=stats, **kw)
     assert stats["path"] == 1 and stats["p1_form"] == 1
+
+
+@pytest.mark.parametrize("flags", [0, qk.GB_ASYNC])
+def test_wide_keys_without_scratch(flags):
+    """A block of a wide-key table takes the one-pass kernel when the two phases' buffers cannot be had,
+    also between blocks that have them."""
+    rng = np.random.default_rng(5)
+    n, block = 300_000, 100_000
+    code = rng.integers(0, 30_000, n)
+    keys, vals = [(code % 211).astype(np.int32), (code // 211).astype(np.int64)], rng.integers(-1000, 1000, n)
+    kn = [rng.random(n) < 0.01, None]
+    aggs = [qk.AGG_SUM, qk.AGG_MIN, qk.AGG_MAX, qk.AGG_COUNT]
+    gb = qk.GPUGroupBy(aggs, [qk.INT, qk.LONG], qk.LONG, 40_000, 1, flags=flags)
+    gb.set_path(1, 0)
+    paths = []
+    for at in range(0, n, block):
+        part = slice(at, at + block)
+        cols = [col(keys[0][part], kn[0][part]), col(keys[1][part]), col(vals[part])]
+        try:
+            if at == 0:
+                qk._abi.call("qk_device_synchronize")
+                qk._abi.call("qk_mem_release_cached")
+                qk.set_memory_limit(qk.memory_stats()[0] + (1 << 20))
+            gb.ProcessBlock([c.data for c in cols[:2]], cols[2].data, block, [c.nulls for c in cols[:2]], None)
+        finally:
+            qk.set_memory_limit(0)
+        paths.append(gb.stats()["path"])
+    got = gb.results_host()
+    gb.close()
+    want = cpu_group_by(aggs, keys, vals, key_nulls=kn)
+    assert paths == [0, 1, 1]
+    for a in range(len(aggs)):
+        maps_close(by_key(got, a), by_key(want, a), rel=0.0)
