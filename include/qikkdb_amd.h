@@ -390,10 +390,12 @@ int qk_gb_describe(qk_groupby h, int32_t* slot_bytes, int64_t* slots, int32_t* l
  * that setting unchanged. */
 int qk_gb_set_tuning(qk_groupby h, int32_t block, int32_t lds_bytes, int32_t wgs_per_cu);
 
-/* Row-kernel path for single-word keys (no reference counterpart): path -1 = automatic
- * (two-phase partitioned aggregation for blocks of at least min_rows rows, the one-pass
- * kernel below that), 0 = always one-pass, 1 = always two-phase.  min_rows < 0 leaves the
- * threshold unchanged.  Results do not depend on the path. */
+/* Row-kernel path (no reference counterpart): path -1 = automatic (two-phase partitioned
+ * aggregation for blocks of at least min_rows rows, the one-pass kernel below that and for
+ * tables whose every key fits a workgroup's LDS), 0 = always one-pass, 1 = always two-phase
+ * where the table allows it.  min_rows < 0 leaves the threshold unchanged.  Keys of more than
+ * one word take the two phases over their slots in the table, and the one-pass kernel when
+ * their buffers cannot be had (no memory, graph capture).  Results do not depend on the path. */
 int qk_gb_set_path(qk_groupby h, int32_t path, int64_t min_rows);
 
 /* Deferred merging on the two-phase path (no reference counterpart).  A table created with
@@ -401,7 +403,8 @@ int qk_gb_set_path(qk_groupby h, int32_t path, int64_t min_rows);
  * once, when the table is next read (qk_gb_get_results, qk_gb_group_count,
  * qk_gb_check_error) or when the buffers are full.  rows: how many rows may be kept
  * (-1 = default: four blocks, at most 2^28 rows; 0 = merge after every block).  The
- * partition buffers take about 24 bytes per kept row. */
+ * partition buffers take about 24 bytes per kept row (and, for keys of more than one word, 4
+ * bytes per row of the largest block). */
 int qk_gb_set_defer_rows(qk_groupby h, int64_t rows);
 
 /* Internal state for tuning (no reference counterpart); waits for the table's work.
@@ -428,6 +431,11 @@ int qk_gb_stats(qk_groupby h, int64_t* out, int32_t n, void* stream);
  * its result with atomics.  A larger query takes two passes: its passing rows are first
  * written to a scratch pool grouped by key chunk, then each chunk is aggregated in LDS by one
  * workgroup (rows that find no room in the pool are aggregated with device atomics).
+ *
+ * A run that reads the table's rows many times over first copies the tiles it touches, ordered
+ * by ts within chunks of 4096 rows, so that a query reads little more than the rows it keeps.
+ * The copy belongs to the engine (20 B per table row, kept between runs, written anew by every
+ * run); without the memory for it the queries read the columns.
  * ====================================================================================== */
 
 typedef struct qk_batch_columns {
@@ -514,8 +522,9 @@ typedef struct qk_serve_config {
     int32_t engines;          /* batch engines: batches running or holding results (0 = 2) */
     int32_t max_batch;        /* most requests per batch (0 = 4096) */
     int64_t memory_cap;       /* projected bytes admitted at once (0 = 200 GB); the engines' row
-                                 pools share the device memory left over it (scratch_rows is
-                                 lowered to fit, QK_OUT_OF_MEMORY when under 2^20 rows each) */
+                                 pools and ts-ordered copies share the device memory left over
+                                 it (the copies at most half of it; scratch_rows is lowered to fit,
+                                 QK_OUT_OF_MEMORY when under 2^20 rows each) */
     double wait_ms;           /* with a batch running, the next one starts when its oldest
                                  request has waited this long (0 = half the last batch's time) */
     qk_batch_tuning tuning;   /* of every engine (tile_rows 0 = defaults, no graph replay) */
